@@ -536,7 +536,8 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(4, 5)
     const float kMagic = 12582912.0f;
     if (wv == 0 && lane < 2 * RS && (lane & (RS - 1)) >= W) red[lane] = 0.0f;   // before the first barrier
 
-    // One row per workgroup (the grid is M).  Two chunk buffers in turn: while
+    // One row per workgroup (the grid is M, tiled outputs: M padded to whole 256-row
+    // tiles).  Two chunk buffers in turn: while
     // pass p is rotated from bufs[p & 1], the wave loads its next pass into the
     // other one, so no register copies carry a prefetch across passes.  Every
     // load is unconditional (a lane past the row end reads the pass's first
@@ -546,6 +547,24 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(4, 5)
     // are left out of the row absmax and store no codes.
     ChunkRegs<DT> bufs[2];
     const int row = blockIdx.x;
+    if constexpr (OUT == OUT_I8T || B6) {
+        // Zero codes in the padding rows of the last 256-row tile, one workgroup
+        // per row: the workgroups of the M data rows wrote them in turn before,
+        // which left a one-row call waiting for one workgroup to clear 255 rows
+        // (M = 1, K = 3072, B6T, kernel trace: 33.8 us, now 2.7).
+        if (row >= M) {
+            if constexpr (B6) {
+                const uint32_t z[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+                for (int k0 = 32 * (wv * 64 + lane); k0 < K; k0 += 32 * 64 * W) b6_store_group(qout, row, K, k0, z);
+            } else {
+                int8_t* tile = qout + (size_t)(row >> 8) * (K >> 6) * I8T_CHUNK;
+                for (int k0 = 16 * (wv * 64 + lane); k0 < K; k0 += 16 * 64 * W)
+                    *reinterpret_cast<uint4*>(tile + (size_t)(k0 >> 6) * I8T_CHUNK + i8t_off(row & 255, (k0 >> 4) & 3)) =
+                        make_uint4(0u, 0u, 0u, 0u);
+            }
+            return;
+        }
+    }
     {
         const int c0 = wv * 64;   // < nchunks: W <= number of passes of a row
         load_regs<DT>(x, (size_t)row * K + (size_t)(c0 + lane < nchunks ? c0 + lane : c0) * kChunk, bufs[0]);
@@ -785,21 +804,11 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(4, 5)
             }
         }
     }
-    if constexpr (OUT == OUT_I8T) {   // zero codes in the padding rows of the last 256-row tile
-        const int mpad = (M + 255) & ~255;
-        for (int prow = M + blockIdx.x; prow < mpad; prow += gridDim.x)
-            for (int k0 = 16 * (wv * 64 + lane); k0 < K; k0 += 16 * 64 * W) {
-                int8_t* chunk = qout + ((size_t)(prow >> 8) * (K >> 6) + (k0 >> 6)) * I8T_CHUNK;
-                *reinterpret_cast<uint4*>(chunk + i8t_off(prow & 255, (k0 >> 4) & 3)) = make_uint4(0u, 0u, 0u, 0u);
-            }
-    }
-    if constexpr (B6) {   // zero codes in the padding rows of the last 256-row tile
-        const int mpad = (M + 255) & ~255;
-        const uint32_t z[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-        for (int prow = M + blockIdx.x; prow < mpad; prow += gridDim.x)
-            for (int k0 = 32 * (wv * 64 + lane); k0 < K; k0 += 32 * 64 * W) b6_store_group(qout, prow, K, k0, z);
-    }
 }
+
+// Workgroups of a launch: one per row, tiled outputs one per padded row.
+template <int OUT>
+static int rq_row_grid(int M) { return OUT == OUT_B6T || OUT == OUT_I8T ? (M + 255) / 256 * 256 : M; }
 
 // Launch shape: a row is np = ceil(K / 1024) passes of 64 lanes; W <= 4 waves
 // of a workgroup share it with P = ceil(np / W) passes each.  Rows of up to 4
@@ -830,7 +839,7 @@ static hipError_t rq_wide_launch(const void* x, int8_t* q, float* s, int M, int 
                        kRowWideWaves * kRowWaveLds + 32 * (int)sizeof(float));
     if (e != hipSuccess) return e;
     const size_t lds = (size_t)W * kRowWaveLds + 32 * sizeof(float);
-    hipLaunchKernelGGL(kern, dim3(M), dim3(64 * W), lds, st, x, q, s, M, K, ls);
+    hipLaunchKernelGGL(kern, dim3(rq_row_grid<OUT>(M)), dim3(64 * W), lds, st, x, q, s, M, K, ls);
     return hipGetLastError();
 }
 
@@ -878,7 +887,7 @@ static hipError_t rq_row_launch(const void* x, int8_t* q, float* s, int M, int K
     // 4608 x 12288 45.4-51.5 against 48.0-54.3 with 3; 16384 x 12288
     // 140.9-153.9 against 153.3-201.4 with 11; 4608 x 3072 runs one row per
     // workgroup either way, 16.8-17.4 us).
-    const int grid = M;
+    const int grid = rq_row_grid<OUT>(M);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * W), lds, st, x, q, s, M, K, ls);
     return hipGetLastError();
 }
