@@ -159,9 +159,12 @@ def dequantize_convrot_w4a4_weight(
 ) -> torch.Tensor:
     """Dequantize packed ConvRot W4A4 weights and rotate back to the original
     basis (reference _int4/eager.py:138-151).  A load-time / diagnostic helper,
-    not on the forward path; computed with torch ops in fp32."""
+    not on the forward path: one kernel on the GPU (csrc/dequant.hip), torch ops
+    in fp32 for anything it does not take."""
     if quant_group_size != _INT4_GROUP_SIZE:
         raise ValueError(f"int4 MMA kernel requires quant_group_size {_INT4_GROUP_SIZE}")
+    if native.dequant_ok(qdata, scales, 4, convrot_groupsize, output_dtype):
+        return native.convrot_dequant(qdata, scales, 4, convrot_groupsize, output_dtype)
     w = _unpack_int4_row_major(qdata).to(torch.float32)
     w = w * scales.to(device=qdata.device, dtype=torch.float32).reshape(-1, 1)
     N, K = w.shape

@@ -2,7 +2,7 @@
 reference's loader, Save and sensitivity nodes import it from
 (``_int4.int8_eager``: int4_ops.py:340, int4_sensitivity.py:67-70,98).  Despite
 the name, quantization runs on the gfx950 kernels; only the load-time
-dequantization helper is torch code.
+dequantization helper has a torch path for other devices.
 
 Numerics: those of the reference eager path (reference _int4/int8_eager.py):
 the exactly rounded block-Hadamard rotation in the input dtype, then
@@ -48,8 +48,11 @@ def dequantize_convrot_w8a8_weight(
     output_dtype: torch.dtype = torch.float32,
 ) -> torch.Tensor:
     """Dequantize int8 ConvRot weights and rotate back to the original basis
-    (reference _int4/int8_eager.py:50-57).  A load-time / diagnostic helper,
-    computed with torch ops in fp32."""
+    (reference _int4/int8_eager.py:50-57).  A load-time / diagnostic helper:
+    one kernel on the GPU (csrc/dequant.hip), torch ops in fp32 for anything it
+    does not take."""
+    if native.dequant_ok(qdata, scales, 8, convrot_groupsize, output_dtype):
+        return native.convrot_dequant(qdata, scales, 8, convrot_groupsize, output_dtype)
     w = qdata.to(torch.float32) * scales.to(qdata.device, torch.float32).reshape(-1, 1)
     N, K = w.shape
     G = convrot_groupsize

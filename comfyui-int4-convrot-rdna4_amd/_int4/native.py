@@ -65,6 +65,7 @@ _SIGNATURES = {
     "cr_convrot_w4a4_linear_bf6_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_bf6_noalloc": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                            + [_vp], _i),
+    "cr_convrot_dequant": ([_vp, _i, _vp, _vp, _i, _i, _i, _i, _vp], _i),
     "cr_max_quant_k": ([], _i),
     "cr_abi_version": ([], _i),
 }
@@ -535,6 +536,43 @@ def int4_convrot_gemm_bf6_lora(a6, w6, x_scale, w_scale, bias, t, up, scale: flo
     odt = {EPI_F32: torch.float32, EPI_BF16: torch.bfloat16, EPI_BF16_EAGER: torch.bfloat16}[epilogue]
     out = torch.empty((M, N), dtype=odt, device=a6.device)
     return _bf6_launch(a6, w6, xs, wsc, b, t, up, R, scale, out, M, N, K, epilogue, nsplit)
+
+
+def is_plain(*ts) -> bool:
+    """Whether one kernel call may stand for a torch composition on these
+    tensors: strided tensors with no transform, trace, dispatch mode or gradient
+    that would have to see the torch operations."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() \
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided
+               and not (t.requires_grad and torch.is_grad_enabled()) for t in ts)
+
+
+def dequant_ok(q, scales, bits: int, convrot_groupsize: int, out_dtype) -> bool:
+    """True when convrot_dequant takes these operands; the torch composition
+    takes every other form (CPU tensors, other devices, groups, types, ranks)."""
+    if not is_plain(q, scales) or q.device.type != "cuda" or q.dim() != 2 or q.dtype != torch.int8:
+        return False
+    N, K = q.shape[0], q.shape[1] * (8 // bits)
+    return (out_dtype in _IN_DTYPE_CODE and convrot_groupsize in (16, 64, 256) and K > 0 and K % convrot_groupsize == 0
+            and N * (K // 16) < 1 << 31 and scales.numel() == N and q.device.index == torch.cuda.current_device()
+            and is_available())
+
+
+def convrot_dequant(q, scales, bits: int, convrot_groupsize: int, out_dtype):
+    """scales[n] * (codes of row n rotated back) -> [N, K]; q packed int4 [N, K/2]
+    (bits 4) or int8 [N, K] (bits 8)."""
+    lib = load_library()
+    q = _aligned(q)
+    s = scales.to(q.device, torch.float32).reshape(-1).contiguous()
+    N, K = q.shape[0], q.shape[1] * (8 // bits)
+    out = torch.empty((N, K), dtype=out_dtype, device=q.device)
+    rc = lib.cr_convrot_dequant(_ptr(q), bits, _ptr(s), _ptr(out), _IN_DTYPE_CODE[out_dtype], N, K, convrot_groupsize,
+                                _stream(q.device))
+    if rc != 0:
+        raise RuntimeError(f"cr_convrot_dequant failed, hipError={rc}")
+    return out
 
 
 # ----------------------------------------------------------------------------

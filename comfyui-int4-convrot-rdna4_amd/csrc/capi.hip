@@ -38,6 +38,8 @@ hipError_t gemm_i8t_launch(const int8_t* X, const int8_t* W, const float* xs, co
                            const float* bias, void* out, int M, int N, int K, int epi, hipStream_t st);
 size_t gemm_bf6_splitk_workspace(int M, int N, int nsplit);
 void gemm_bf6_tile(int M, int N, int K, int nsplit, int* bm, int* bn);
+hipError_t dequant_launch(const void* q, int bits, const float* s, void* out, int odt, int N, int K, int G,
+                          hipStream_t st);
 hipError_t gemm_splitk_launch(const int8_t* Xp, const int8_t* Wp, const float* xs, const float* ws, float* accum,
                               int M, int N, int K, int nsplit, hipStream_t st);
 }  // namespace convrot
@@ -393,6 +395,14 @@ API int cr_convrot_w4a4_linear_bf6_noalloc(const void* x, int in_dtype, const vo
     if (e != hipSuccess) return (int)e;
     return linear_bf6_run(x, in_dtype, W6, wscale, bias, bias_dtype, D, U, R, scale, out, epilogue, M, N, K, G, p, ws,
                           stream);
+}
+
+API int cr_convrot_dequant(const void* q, int bits, const void* scale, void* out, int out_dtype, int N, int K, int G,
+                           void* stream) {
+    if ((bits != 4 && bits != 8) || !(G == 16 || G == 64 || G == 256) || out_dtype < 0 || out_dtype > 2) return -1;
+    if (N < 0 || K <= 0 || K % G != 0 || (long long)N * (K / 16) >= (1ll << 31)) return -1;
+    return (int)convrot::dequant_launch(q, bits, reinterpret_cast<const float*>(scale), out, out_dtype, N, K, G,
+                                        reinterpret_cast<hipStream_t>(stream));
 }
 
 API int cr_max_quant_k(void) { return convrot::rotquant_max_k(); }

@@ -340,6 +340,19 @@ int cr_int8_convrot_gemm_i8t(const void* X, const void* W, const void* xscale, c
 /* Largest K accepted by the quantization entry points. */
 int cr_max_quant_k(void);
 
+/*
+ * Dequantize ConvRot weights back to the original basis: out[n, :] =
+ * scale[n] * (q[n, :] rotated by H_G), q packed int4 [N, K/2] (bits 4) or int8
+ * [N, K] (bits 8), both 16-byte aligned, scale f32 [N], out [N, K] f32, bf16 or
+ * f16 (out_dtype as the input dtype codes).  The rotation of the codes is an
+ * exact integer sum; the scale is multiplied in with one fp32 rounding, then
+ * the output type's.  G in {16, 64, 256}, K % G == 0, N K / 16 < 2^31.
+ * Replaces the torch dequantizers of _int4/eager.py:138-151 and
+ * _int4/int8_eager.py:50-57.
+ */
+int cr_convrot_dequant(const void* q, int bits, const void* scale, void* out, int out_dtype, int N, int K, int G,
+                       void* stream);
+
 /* ABI version of this library (increments on any signature change). */
 int cr_abi_version(void);
 
