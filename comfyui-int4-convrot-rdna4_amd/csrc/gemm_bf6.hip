@@ -23,69 +23,64 @@ namespace convrot {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-// codes of nibbles base .. base+7 (two's complement int4), 6 bits each
-constexpr uint64_t bf6_nibble_table(int base) {
-    uint64_t t = 0;
-    for (int i = 0; i < 8; ++i) {
-        const int n = base + i;
-        t |= (uint64_t)bf6_code_of_int(n >= 8 ? n - 16 : n) << (6 * i);
-    }
-    return t;
-}
-
-__device__ __forceinline__ uint32_t bf6_of_nibble(uint32_t n) {
-    constexpr uint64_t LO = bf6_nibble_table(0), HI = bf6_nibble_table(8);
-    const uint64_t t = (n & 8) ? HI : LO;
-    return (uint32_t)(t >> ((n & 7) * 6)) & 63u;
+// BF6 codes of the four two's complement nibbles in the low halves of the bytes
+// of b: the sign to bit 5, the magnitude 0..8 below (bf6_code_of_int).
+__device__ __forceinline__ uint32_t bf6_of_nibbles(uint32_t b) {
+    const uint32_t m = b & 0x08080808u, s = m >> 3;
+    return ((b ^ ((m << 1) - s)) + s) | (m << 2);     // n ^ 15 + 1 where negative: no carry leaves a byte
 }
 
 // 32 packed nibbles (element e = nibble e of the 16 bytes, low nibble first)
 // -> one 6-dword bf6 operand
 __device__ __forceinline__ void encode_group(uint4 p, uint32_t (&d)[6]) {
     const uint32_t w[4] = {p.x, p.y, p.z, p.w};
+    uint32_t h[8];                                    // 24-bit runs of four codes
 #pragma unroll
-    for (int i = 0; i < 6; ++i) d[i] = 0;
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t ev = bf6_of_nibbles(w[i] & 0x0f0f0f0fu), od = bf6_of_nibbles((w[i] >> 4) & 0x0f0f0f0fu);
+        const uint32_t a = (ev & 0x00ff00ffu) | ((od & 0x00ff00ffu) << 6);                 // codes 0,1 and 4,5
+        const uint32_t b = ((ev >> 8) & 0x00ff00ffu) | (((od >> 8) & 0x00ff00ffu) << 6);   // codes 2,3 and 6,7
+        h[2 * i] = (a & 0xfffu) | ((b & 0xfffu) << 12);
+        h[2 * i + 1] = (a >> 16) | ((b >> 16) << 12);
+    }
 #pragma unroll
-    for (int e = 0; e < 32; ++e) {
-        const uint32_t code = bf6_of_nibble((w[e >> 3] >> ((e & 7) * 4)) & 15u);
-        const int bit = 6 * e;
-        d[bit >> 5] |= code << (bit & 31);
-        if ((bit & 31) > 26) d[(bit >> 5) + 1] |= code >> (32 - (bit & 31));
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t* x = h + 4 * i;
+        d[3 * i] = x[0] | (x[1] << 24);
+        d[3 * i + 1] = (x[1] >> 8) | (x[2] << 16);
+        d[3 * i + 2] = (x[2] >> 16) | (x[3] << 8);
     }
 }
 
-// packed int4 [rows, K/2] -> B6T; one thread per (row, 128-k block) of the
-// padded matrix, consecutive threads on consecutive rows of one chunk.
+// packed int4 [rows, K/2] -> B6T.  HBM-bound: K/2 bytes in, 3K/4 out per row.
+// A thread encodes group g of rows r and r + 32 of a tile pair, so that it owns
+// a whole 16-byte Q piece, and a wave's 16 rows x 4 groups write three runs of
+// 1 KB (the P rows of either tile, the Q rows); a workgroup's four waves take
+// consecutive 128-k blocks of the same rows, 256 consecutive bytes of each.
+// 12288 x 3072 on MI355X (47 MB, kernel trace): 13.1 us, against 18.7 with one
+// thread per (row, block), whose stores were 16 and 8 bytes apart by 64 and
+// whose codes came one by one from a 64-bit table.
 __global__ __launch_bounds__(256) void int4_to_bf6t_kernel(const uint8_t* __restrict__ src,
                                                            uint8_t* __restrict__ dst, int rows, int K) {
     const int nkb = K / 128;
-    const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
-    const int tiles = (rows + 255) / 256;
-    if (id >= (long long)tiles * nkb * 256) return;
-    const int r = (int)(id & 255);
-    const long long tk = id >> 8;                        // tile * nkb + kb
-    const int tile = (int)(tk / nkb), kb = (int)(tk % nkb);
+    const int kb = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (kb >= nkb) return;
+    const int lane = threadIdx.x & 63;
+    const int tile = blockIdx.x >> 3, part = blockIdx.x & 7;      // part: tile pair (2 bits), upper / lower 16 rows
+    const int g = lane & 3;
+    const int r = (part >> 1) * 64 + (part & 1) * 16 + (lane >> 2);   // row of the even tile
     const int row = tile * 256 + r;
-    uint4 in[4] = {};
-    if (row < rows) {
-        const uint4* s = reinterpret_cast<const uint4*>(src + (size_t)row * (K / 2) + (size_t)kb * 64);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) in[g] = s[g];
-    }
-    uint8_t* d = dst + (size_t)tk * B6_CHUNK;
-    const bool odd = b6_odd_tile(r);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        uint32_t c[6];
-        encode_group(in[g], c);
-        if (!odd) {
-            *reinterpret_cast<uint4*>(d + b6_p_off(r, g)) = make_uint4(c[0], c[1], c[2], c[3]);
-            *reinterpret_cast<uint2*>(d + b6_q_off(r, g)) = make_uint2(c[4], c[5]);
-        } else {
-            *reinterpret_cast<uint4*>(d + b6_p_off(r, g)) = make_uint4(c[2], c[3], c[4], c[5]);
-            *reinterpret_cast<uint2*>(d + b6_q_off(r, g) + 8) = make_uint2(c[0], c[1]);
-        }
-    }
+    const uint8_t* s = src + (size_t)row * (K / 2) + (size_t)kb * 64 + g * 16;
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    const uint4 in0 = row < rows ? *reinterpret_cast<const uint4*>(s) : zero;
+    const uint4 in1 = row + 32 < rows ? *reinterpret_cast<const uint4*>(s + (size_t)16 * K) : zero;
+    uint32_t c[6], o[6];
+    encode_group(in0, c);
+    encode_group(in1, o);
+    uint8_t* d = dst + ((size_t)tile * nkb + kb) * B6_CHUNK;
+    *reinterpret_cast<uint4*>(d + b6_p_off(r, g)) = make_uint4(c[0], c[1], c[2], c[3]);
+    *reinterpret_cast<uint4*>(d + b6_p_off(r + 32, g)) = make_uint4(o[2], o[3], o[4], o[5]);
+    *reinterpret_cast<uint4*>(d + b6_q_off(r, g)) = make_uint4(c[4], c[5], o[0], o[1]);
 }
 
 // int4 value of a B6T code (bf6_code_of_int: |q| in bits 0..4, sign in bit 5;
@@ -783,8 +778,7 @@ static hipError_t launch_bf6(const uint8_t* A6, const uint8_t* W6, const float* 
 
 hipError_t int4_to_bf6_launch(const void* src, void* dst, int rows, int K, hipStream_t st) {
     if (rows == 0) return hipSuccess;
-    const long long n = (long long)((rows + 255) / 256) * (K / 128) * 256;
-    hipLaunchKernelGGL(int4_to_bf6t_kernel, dim3((unsigned)(n / 256)), dim3(256), 0, st,
+    hipLaunchKernelGGL(int4_to_bf6t_kernel, dim3((unsigned)((rows + 255) / 256) * 8, (K / 128 + 3) / 4), dim3(256), 0, st,
                        reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), rows, K);
     return hipGetLastError();
 }
