@@ -31,6 +31,7 @@ hipError_t gemm_bf6_launch(const void* A6, const void* W6, const float* xs, cons
                            int bias_dt, const void* t, const void* U, int R, float scale, void* out, int M, int N,
                            int K, int epi, int nsplit, void* workspace, hipStream_t st);
 int gemm_bf6_choose_nsplit(int M, int N, int K);
+void gemm_bf6_direct_tile(int M, int N, int K, int* bm, int* bn);
 hipError_t rotquant_i8t_launch(const void* x, int in_dtype, int8_t* q, float* s, int M, int K, int G,
                                hipStream_t st);
 hipError_t int8_to_i8t_launch(const void* src, void* dst, int rows, int K, hipStream_t st);
@@ -281,8 +282,11 @@ LinPlan lin_plan(int M, int N, int K, int R) {
     LinPlan p{};
     const size_t rows = (size_t)((M + 255) / 256) * 256;
     p.nsplit = convrot::gemm_bf6_choose_nsplit(M, N, K);
+    int bm = 0, bn = 0;
+    convrot::gemm_bf6_direct_tile(M, N, K, &bm, &bn);
+    if (bm != 0) p.nsplit = 1;      // the direct kernel splits k inside its workgroups
     p.part = 0;
-    const size_t split_bytes = convrot::gemm_bf6_splitk_workspace(M, N, p.nsplit);
+    const size_t split_bytes = convrot::gemm_bf6_splitk_workspace(M, N, convrot::gemm_bf6_choose_nsplit(M, N, K));
     p.a6 = al256(split_bytes > kSplitCounterBytes ? split_bytes : kSplitCounterBytes);
     p.xs = p.a6 + al256(rows * (size_t)K / 4 * 3);
     p.t = p.xs + al256((size_t)M * 4);

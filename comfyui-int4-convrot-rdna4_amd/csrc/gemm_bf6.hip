@@ -693,6 +693,10 @@ __global__ __launch_bounds__(64 * B6R_WAVES) void w4a4_bf6_splitk_reduce_kernel(
 
 bool gemm_bf6_small_tiles(int M, int N, int K);
 int gemm_bf6_small_shape(int M, int N, int K, int nsplit);
+void gemm_bf6_direct_tile(int M, int N, int K, int* bm, int* bn);
+hipError_t gemm_bf6_direct_launch(const uint8_t* A, const uint8_t* B, const float* xs, const float* ws,
+                                  const void* bias, int bias_dt, void* out, int M, int N, int K, const LoraArgs& la,
+                                  int epi, hipStream_t st);
 
 // One launch of the small kernel of shape (UA, UB) with NST stages, split nsplit ways.
 template <int EPI, int LR, int UA, int UB, int NST = B6S_STAGES>
@@ -798,8 +802,11 @@ hipError_t gemm_bf6_launch(const void* A6, const void* W6, const float* xs, cons
     if (M == 0 || N == 0) return hipSuccess;
     const uint8_t* a = reinterpret_cast<const uint8_t*>(A6);
     const uint8_t* w = reinterpret_cast<const uint8_t*>(W6);
+    int dbm = 0, dbn = 0;
+    if (nsplit <= 1) gemm_bf6_direct_tile(M, N, K, &dbm, &dbn);
     if (t == nullptr) {
         const LoraArgs none{nullptr, nullptr, 0, 0.0f};
+        if (dbm) return gemm_bf6_direct_launch(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, epi, st);
         switch (epi) {
             case EPI_F32: return launch_bf6<EPI_F32, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
             case EPI_BF16: return launch_bf6<EPI_BF16, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
@@ -810,6 +817,7 @@ hipError_t gemm_bf6_launch(const void* A6, const void* W6, const float* xs, cons
     }
     const LoraArgs la{reinterpret_cast<const __bf16*>(t), reinterpret_cast<const __bf16*>(U), R, scale};
     if (R % 32 != 0 || R < 32 || R > 128) return hipErrorInvalidValue;
+    if (dbm) return gemm_bf6_direct_launch(a, w, xs, ws, bias, bias_dt, out, M, N, K, la, epi, st);
 #define BF6_LORA_CASE(LRV)                                                                                      \
     case LRV:                                                                                                   \
         switch (epi) {                                                                                          \
@@ -869,6 +877,9 @@ int gemm_bf6_small_shape(int M, int N, int K, int nsplit) {
 
 // The workgroup tile (rows of A x rows of B) of a bf6 GEMM launch.
 void gemm_bf6_tile(int M, int N, int K, int nsplit, int* bm, int* bn) {
+    *bm = 0;
+    if (nsplit <= 1) gemm_bf6_direct_tile(M, N, K, bm, bn);
+    if (*bm) return;
     if (!gemm_bf6_small_tiles(M, N, K)) { *bm = B6_BM; *bn = B6_BN; return; }
     *bm = 128;
     *bn = gemm_bf6_small_shape(M, N, K, nsplit) == SMALL_128x192 ? 192 : 128;

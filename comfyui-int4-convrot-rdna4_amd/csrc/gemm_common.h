@@ -15,7 +15,21 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // EPI_ATOMIC_ACC: the k-split partial of the packed split-K entry point; the
 // exact integer accumulator of the workgroup's k range is added atomically
 // into an int32 [M, N] buffer (integer sums are exact in any order).
-enum : int { EPI_F32 = 0, EPI_BF16 = 1, EPI_BF16_EAGER = 2, EPI_ACC = 3, EPI_ATOMIC_ACC = 4 };
+enum : int { EPI_F32 = 0, EPI_BF16 = 1, EPI_BF16_EAGER = 2, EPI_ACC = 3, EPI_ATOMIC_ACC = 4,
+             EPI_F16 = 5 };
+
+// bytes of an output element
+template <int EPI> constexpr int epi_bytes = EPI == EPI_BF16 || EPI == EPI_BF16_EAGER || EPI == EPI_F16 ? 2 : 4;
+
+// two outputs of a 16-bit type, packed (EPI_F16: the f32 epilogue's value
+// rounded once to f16, past its range to infinity as a cast does)
+template <int EPI>
+__device__ __forceinline__ uint32_t pack_out2(float a, float b) {
+    if constexpr (EPI == EPI_F16)
+        return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
+    else
+        return pack_bf16x2(a, b);
+}
 
 __device__ __forceinline__ float bf16r(float f) { return round_to_dt<DT_BF16>(f); }
 
@@ -207,8 +221,8 @@ __device__ __forceinline__ void epilogue_lds(const AccV (&acc)[FMT][FNT], const 
                                              int row0, int col0, int lane, const LoraArgs& la, uint8_t* scr,
                                              const uint8_t* tu_lds = nullptr) {
     constexpr bool LORA = LR != 0;
-    constexpr bool PRE = LR == 1 && (EPI == EPI_BF16 || EPI == EPI_BF16_EAGER);
-    constexpr int ES = (EPI == EPI_BF16 || EPI == EPI_BF16_EAGER) ? 2 : 4;
+    constexpr bool PRE = LR == 1 && epi_bytes<EPI> == 2;
+    constexpr int ES = epi_bytes<EPI>;
     constexpr int RB = FNT * 32 * ES;                // bytes of one wave-tile row
     constexpr int RS = RB + 16;                      // padded LDS row stride
     // One 32-row tile per staging pass: the stores of a pass drain while the next
@@ -358,7 +372,7 @@ __device__ __forceinline__ void epilogue_lds(const AccV (&acc)[FMT][FNT], const 
                         if constexpr (ES == 4) {
                             *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
                         } else {
-                            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_out2<EPI>(v[0], v[1]), pack_out2<EPI>(v[2], v[3]));
                         }
                     }
                 }
