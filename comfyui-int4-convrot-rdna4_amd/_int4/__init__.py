@@ -281,11 +281,16 @@ def convrot_w4a4_linear(
         raise ValueError(f"wscales has {wscales.numel()} elements, the weight has N={N} rows")
     if bias is not None and bias.numel() != N:
         raise ValueError(f"bias has {bias.numel()} elements, the weight has N={N} rows")
-    if bf6_path_ok(K) and x2d.is_cuda and (lora is None or x2d.dtype in (torch.bfloat16, torch.float16)):
+    packed = not bf6_path_ok(K)
+    if (not packed or (K % 64 == 0 and qweight.dtype == torch.int8)) and x2d.is_cuda \
+            and (lora is None or x2d.dtype in (torch.bfloat16, torch.float16)):
         # the whole linear in one library call (same kernels, same bits as the steps below)
-        w6 = qweight_bf6 if qweight_bf6 is not None else prepare_convrot_w4a4_weight_bf6(qweight)
-        if w6.shape != (native.bf6_rows(N), K // 4 * 3):
-            raise ValueError(f"qweight_bf6 of shape {tuple(w6.shape)} does not encode a [{N}, {K}] weight")
+        if packed:
+            w = native._aligned(qweight)
+        else:
+            w = qweight_bf6 if qweight_bf6 is not None else prepare_convrot_w4a4_weight_bf6(qweight)
+            if w.shape != (native.bf6_rows(N), K // 4 * 3):
+                raise ValueError(f"qweight_bf6 of shape {tuple(w.shape)} does not encode a [{N}, {K}] weight")
         wsc = wscales if wscales.dtype == torch.float32 and wscales.is_contiguous() else \
             wscales.reshape(-1).to(torch.float32).contiguous()
         # the bias is read as stored (f32 / bf16 / f16): no conversion launch per call
@@ -295,10 +300,13 @@ def convrot_w4a4_linear(
             b32 = b32.contiguous()
         down = up = None
         if lora is not None:
-            down, up = lora
-        native._check_cuda(x2d, w6, wsc, b32, down, up)
-        out = native.convrot_w4a4_linear_bf6(native._aligned(x2d), w6, wsc, b32, down, up, 1.0, epi,
-                                             convrot_groupsize, N)
+            down, up = native._aligned(lora[0]), native._aligned(lora[1])
+        native._check_cuda(x2d, w, wsc, b32, down, up)
+        x2d = native._aligned(x2d)
+        if packed:
+            out = native.convrot_w4a4_linear_packed(x2d, w, wsc, b32, down, up, 1.0, epi, convrot_groupsize)
+        else:
+            out = native.convrot_w4a4_linear_bf6(x2d, w, wsc, b32, down, up, 1.0, epi, convrot_groupsize, N)
         if out.dtype != x.dtype:
             out = out.to(x.dtype)
         return out.reshape(*orig_shape[:-1], N)
@@ -395,12 +403,17 @@ def convrot_w8a8_linear(
     if x2d.dtype not in native._IN_DTYPE_CODE:
         x2d = x2d.to(torch.float32)
     out_dtype = x.dtype if x.dtype in _NATIVE_OUT else torch.float32
-    M, N = x2d.shape[0], qweight.shape[0]
+    N = qweight.shape[0]
     if i8t_path_ok(x2d.shape[1]) and x2d.is_cuda:
         w8t = qweight_i8t if qweight_i8t is not None else prepare_convrot_w8a8_weight_i8t(qweight)
-        a8t, x_scale = native.convrot_quant_int8_i8t(x2d, convrot_groupsize)
+        # the bias is read as stored (f32 / bf16 / f16): no conversion launch per call
+        b = bias if bias is None or bias.dtype in native._IN_DTYPE_CODE else bias.to(torch.float32)
+        b = None if b is None else b.contiguous()
+        wsc = wscales.to(torch.float32).contiguous()
+        native._check_cuda(w8t, wsc, b)
         epi = native.EPI_F32 if out_dtype == torch.float32 else native.EPI_BF16
-        out = native.int8_convrot_gemm_i8t(a8t, w8t, x_scale, wscales, bias, epi, M, N)
+        out = native.convrot_w8a8_linear_i8t(native._aligned(x2d), native._aligned(w8t), wsc, b, epi,
+                                             convrot_groupsize, N)
     else:
         qact, x_scale = native.convrot_quant_int8(x2d, convrot_groupsize)
         out = native.int8_convrot_gemm(qact, qweight, x_scale, wscales, bias, out_dtype)

@@ -16,8 +16,8 @@ from concurrent.futures import ThreadPoolExecutor
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _PKG = os.path.dirname(_HERE)
 _CSRC = os.path.join(_PKG, "csrc")
-SOURCES = ("rotquant.hip", "gemm.hip", "gemm_bf6.hip", "gemm_bf6_direct.hip", "lora.hip", "dequant.hip", "capi.hip")
-HEADERS = ("common.h", "gemm_common.h", "gemm_direct.h", "b6t_layout.h")
+SOURCES = ("rotquant.hip", "gemm.hip", "gemm_bf6.hip", "gemm_bf6_direct.hip", "gemm_int.hip", "lora.hip", "dequant.hip", "capi.hip")
+HEADERS = ("common.h", "gemm_common.h", "gemm_direct.h", "gemm_int.h", "b6t_layout.h")
 ARCH = "gfx950"
 
 

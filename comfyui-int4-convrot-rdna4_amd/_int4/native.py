@@ -65,6 +65,11 @@ _SIGNATURES = {
     "cr_convrot_w4a4_linear_bf6_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_bf6_noalloc": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                            + [_vp], _i),
+    "cr_convrot_w8a8_linear_i8t": ([_vp, _i, _vp, _vp, _vp, _i, _vp] + [_i] * 5 + [_vp, ctypes.c_size_t, _vp], _i),
+    "cr_convrot_w8a8_linear_i8t_workspace": ([_i, _i, _i], ctypes.c_size_t),
+    "cr_convrot_w4a4_linear_packed": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
+                                      + [_vp, ctypes.c_size_t, _vp], _i),
+    "cr_convrot_w4a4_linear_packed_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
     "cr_convrot_dequant": ([_vp, _i, _vp, _vp, _i, _i, _i, _i, _vp], _i),
     "cr_max_quant_k": ([], _i),
     "cr_abi_version": ([], _i),
@@ -743,4 +748,47 @@ def convrot_w4a4_linear_bf6(x2d, w6, w_scale, bias, down, up, scale: float, epil
                                         M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
     if rc != 0:
         raise RuntimeError(f"cr_convrot_w4a4_linear_bf6 failed, hipError={rc}")
+    return out
+
+
+def convrot_w4a4_linear_packed(x2d, qweight, w_scale, bias, down, up, scale: float, epilogue: int,
+                               convrot_groupsize: int):
+    """convrot_w4a4_linear_bf6 on the packed int4 weight [N, K/2] itself, for the
+    widths B6T does not hold (K % 64 == 0): one library call."""
+    lib = load_library()
+    M, K = x2d.shape
+    N = qweight.shape[0]
+    odt = {EPI_F32: torch.float32, EPI_BF16: torch.bfloat16, EPI_BF16_EAGER: torch.bfloat16}[epilogue]
+    out = torch.empty((M, N), dtype=odt, device=x2d.device)
+    R = 0 if down is None else down.shape[0]
+    nbytes = lib.cr_convrot_w4a4_linear_packed_workspace(M, N, K, R)
+    st = _stream(x2d.device)
+    ws = _workspace(x2d.device, st, nbytes)
+    bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
+    rc = lib.cr_convrot_w4a4_linear_packed(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(qweight), _ptr(w_scale),
+                                           _ptr(bias), bdt, _ptr(down), _ptr(up), R, scale, _ptr(out), epilogue,
+                                           M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    if rc != 0:
+        raise RuntimeError(f"cr_convrot_w4a4_linear_packed failed, hipError={rc}")
+    return out
+
+
+def convrot_w8a8_linear_i8t(x2d, w8t, w_scale, bias, epilogue: int, convrot_groupsize: int, N: int):
+    """The whole W8A8 linear on an I8T weight in one library call; bias [N] f32 /
+    bf16 / f16 as stored, or None; epilogue 0 (f32) or 1 (bf16)."""
+    lib = load_library()
+    M, K = x2d.shape
+    if w8t.dtype != torch.int8:
+        raise ValueError("I8T operands must be int8")
+    if w8t.shape[1] != K or w8t.shape[0] != i8t_rows(N):
+        raise ValueError(f"I8T operand shape {tuple(w8t.shape)} does not match N={N}, K={K}")
+    out = torch.empty((M, N), dtype=torch.float32 if epilogue == EPI_F32 else torch.bfloat16, device=x2d.device)
+    nbytes = lib.cr_convrot_w8a8_linear_i8t_workspace(M, N, K)
+    st = _stream(x2d.device)
+    ws = _workspace(x2d.device, st, nbytes)
+    bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
+    rc = lib.cr_convrot_w8a8_linear_i8t(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w8t), _ptr(w_scale), _ptr(bias),
+                                        bdt, _ptr(out), epilogue, M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    if rc != 0:
+        raise RuntimeError(f"cr_convrot_w8a8_linear_i8t failed, hipError={rc}")
     return out

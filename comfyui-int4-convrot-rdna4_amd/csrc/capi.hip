@@ -2,7 +2,7 @@
 // include/convrot_mi355x.h.
 
 #include "../../include/convrot_mi355x.h"
-#include "common.h"
+#include "gemm_common.h"
 
 namespace convrot {
 hipError_t rotquant_launch(const void* x, int in_dtype, const void* noise, int8_t* q, float* s,
@@ -35,8 +35,11 @@ void gemm_bf6_direct_tile(int M, int N, int K, int* bm, int* bn);
 hipError_t rotquant_i8t_launch(const void* x, int in_dtype, int8_t* q, float* s, int M, int K, int G,
                                hipStream_t st);
 hipError_t int8_to_i8t_launch(const void* src, void* dst, int rows, int K, hipStream_t st);
-hipError_t gemm_i8t_launch(const int8_t* X, const int8_t* W, const float* xs, const float* ws,
-                           const float* bias, void* out, int M, int N, int K, int epi, hipStream_t st);
+hipError_t gemm_i8t_launch(const int8_t* X, const int8_t* W, const float* xs, const float* ws, const void* bias,
+                           int bias_dt, void* out, int M, int N, int K, int epi, void* workspace, hipStream_t st);
+size_t gemm_i8t_workspace(int M, int N, int K);
+hipError_t gemm_p4_launch(const int8_t* Xp, const int8_t* Wp, const float* xs, const float* ws, const void* bias,
+                          int bias_dt, void* out, int M, int N, int K, const LoraArgs& la, int epi, hipStream_t st);
 size_t gemm_bf6_splitk_workspace(int M, int N, int nsplit);
 void gemm_bf6_tile(int M, int N, int K, int nsplit, int* bm, int* bn);
 hipError_t dequant_launch(const void* q, int bits, const float* s, void* out, int odt, int N, int K, int G,
@@ -262,7 +265,7 @@ API int cr_int8_convrot_gemm_i8t(const void* X, const void* W, const void* xscal
     if (epilogue != 0 && epilogue != 1 && epilogue != 3) return -1;
     return (int)convrot::gemm_i8t_launch(reinterpret_cast<const int8_t*>(X), reinterpret_cast<const int8_t*>(W),
                                          reinterpret_cast<const float*>(xscale), reinterpret_cast<const float*>(wscale),
-                                         reinterpret_cast<const float*>(bias), out, M, N, K, epilogue,
+                                         bias, convrot::DT_F32, out, M, N, K, epilogue, nullptr,
                                          reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -353,6 +356,81 @@ API int cr_convrot_w4a4_linear_bf6(const void* x, int in_dtype, const void* W6, 
     if (workspace == nullptr || workspace_bytes < p.total) return -1;
     return linear_bf6_run(x, in_dtype, W6, wscale, bias, bias_dtype, D, U, R, scale, out, epilogue, M, N, K, G, p,
                           workspace, stream);
+}
+
+// ---------------------------------------------------------------------------
+// The linears of widths and precisions off the bf6 path, whole, in one call:
+// rotate + quantize x, the LoRA down projection, the GEMM with the bias read as
+// stored.  Workspace as LinPlan: the counters and split partials, the codes, the
+// row scales, t, the LoRA partials.
+// ---------------------------------------------------------------------------
+static LinPlan int_plan(int bits, int M, int N, int K, int R) {
+    LinPlan p{};
+    const size_t split = bits == 8 ? convrot::gemm_i8t_workspace(M, N, K) : 0;
+    p.nsplit = split > 0 ? 2 : 1;   // whether the GEMM splits
+    p.a6 = al256(split > kSplitCounterBytes ? split : kSplitCounterBytes);
+    const size_t codes = bits == 8 ? (size_t)((M + 255) / 256) * 256 * K : (size_t)M * K / 2;
+    p.xs = p.a6 + al256(codes);
+    p.t = p.xs + al256((size_t)M * 4);
+    p.lpart = p.t + al256((size_t)M * R * 2);
+    p.total = p.lpart + (R > 0 ? al256(convrot::lora_part_bytes(M, K, R)) : 0);
+    return p;
+}
+
+API size_t cr_convrot_w8a8_linear_i8t_workspace(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || !i8t_k_ok(K)) return 0;
+    return int_plan(8, M, N, K, 0).total;
+}
+
+API int cr_convrot_w8a8_linear_i8t(const void* x, int in_dtype, const void* W8, const void* wscale, const void* bias,
+                                   int bias_dtype, void* out, int epilogue, int M, int N, int K, int G,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
+    if (!quant_args_ok(in_dtype, M, K, G) || !i8t_k_ok(K) || K > convrot::rotquant_b6_max_k() || N < 0) return -1;
+    if (bias_dtype < 0 || bias_dtype > 2 || (epilogue != 0 && epilogue != 1)) return -1;
+    if (M == 0 || N == 0) return 0;
+    const LinPlan p = int_plan(8, M, N, K, 0);
+    if (workspace == nullptr || workspace_bytes < p.total) return -1;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
+    int8_t* q = reinterpret_cast<int8_t*>(ws + p.a6);
+    float* xs = reinterpret_cast<float*>(ws + p.xs);
+    hipError_t e = convrot::rotquant_i8t_launch(x, in_dtype, q, xs, M, K, G, st);
+    if (e != hipSuccess) return (int)e;
+    return (int)convrot::gemm_i8t_launch(q, reinterpret_cast<const int8_t*>(W8), xs,
+                                         reinterpret_cast<const float*>(wscale), bias, bias_dtype, out, M, N, K,
+                                         epilogue, p.nsplit > 1 ? workspace : nullptr, st);
+}
+
+API size_t cr_convrot_w4a4_linear_packed_workspace(int M, int N, int K, int R) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || K >= 131072 || R < 0) return 0;
+    return int_plan(4, M, N, K, R).total;
+}
+
+API int cr_convrot_w4a4_linear_packed(const void* x, int in_dtype, const void* Wp, const void* wscale,
+                                      const void* bias, int bias_dtype, const void* D, const void* U, int R,
+                                      float scale, void* out, int epilogue, int M, int N, int K, int G,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+    if (!quant_args_ok(in_dtype, M, K, G) || K % 64 != 0 || N < 0) return -1;
+    if (bias_dtype < 0 || bias_dtype > 2 || epilogue < 0 || epilogue > 2) return -1;
+    if (R != 0 && (!lora_rank_ok(R) || D == nullptr || U == nullptr || in_dtype == 0)) return -1;
+    if (M == 0 || N == 0) return 0;
+    const LinPlan p = int_plan(4, M, N, K, R);
+    if (workspace == nullptr || workspace_bytes < p.total) return -1;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
+    int8_t* q = reinterpret_cast<int8_t*>(ws + p.a6);
+    float* xs = reinterpret_cast<float*>(ws + p.xs);
+    hipError_t e = convrot::rotquant_launch(x, in_dtype, nullptr, q, xs, M, K, G, st);
+    if (e != hipSuccess) return (int)e;
+    convrot::LoraArgs la{nullptr, nullptr, 0, 0.0f};
+    if (R != 0) {
+        e = convrot::lora_down_launch(x, in_dtype, D, ws + p.t, M, K, R,
+                                      convrot::lora_part_bytes(M, K, R) > 0 ? reinterpret_cast<float*>(ws + p.lpart) : nullptr, st);
+        if (e != hipSuccess) return (int)e;
+        la = convrot::LoraArgs{reinterpret_cast<const __bf16*>(ws + p.t), reinterpret_cast<const __bf16*>(U), R, scale};
+    }
+    return (int)convrot::gemm_p4_launch(q, reinterpret_cast<const int8_t*>(Wp), xs, reinterpret_cast<const float*>(wscale),
+                                        bias, bias_dtype, out, M, N, K, la, epilogue, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -31,6 +31,9 @@
 
 namespace convrot {
 
+hipError_t gemm_p4_launch(const int8_t* Xp, const int8_t* Wp, const float* xs, const float* ws, const void* bias,
+                          int bias_dt, void* out, int M, int N, int K, const LoraArgs& la, int epi, hipStream_t st);
+
 constexpr int TBM = 256, TBN = 256;  // workgroup tile
 constexpr int TBK = 128;             // k values per LDS block
 constexpr int ROWB = TBK / 2;        // packed bytes per row per block (64)
@@ -196,7 +199,7 @@ constexpr int P_LDS_BYTES = P_STAGES * P_STAGE_BYTES + EPI_SCALE_FLOATS * 4;
 template <int EPI, int WN, bool LORA, bool I8, bool TM = false>
 __global__ __launch_bounds__(128 * WN) void w4a4_gemm_pipe_kernel(
         const int8_t* __restrict__ Xp, const int8_t* __restrict__ Wp,
-        const float* __restrict__ xs, const float* __restrict__ ws, const float* __restrict__ bias,
+        const float* __restrict__ xs, const float* __restrict__ ws, const void* __restrict__ bias, int bias_dt,
         void* __restrict__ out, int M, int N, int K, LoraArgs lora, int gm) {
     extern __shared__ __attribute__((aligned(16))) uint8_t plds[];
 
@@ -219,7 +222,7 @@ __global__ __launch_bounds__(128 * WN) void w4a4_gemm_pipe_kernel(
     const int kb_begin = (int)((long long)blockIdx.y * nkb_all / gridDim.y);
     const int nkb = (int)((long long)(blockIdx.y + 1) * nkb_all / gridDim.y) - kb_begin;
     float* sc = reinterpret_cast<float*>(plds + P_STAGES * P_STAGE_BYTES);
-    stage_scales(sc, xs, ws, bias, M, N, m0, n0, tid, 128 * WN);   // visible after the loop's first barrier
+    stage_scales(sc, xs, ws, bias, bias_dt, M, N, m0, n0, tid, 128 * WN);   // visible after the loop's first barrier
 
     static_assert(!TM || (I8 && WN == 4), "I8T operands: W8A8, 8 waves");
     // DMA source rows / chunks for this lane's P_LOADS instructions (fixed per tile)
@@ -437,8 +440,8 @@ __global__ __launch_bounds__(128 * WN) void w4a4_gemm_pipe_kernel(
 // workgroups per tile, at most one split per k block.
 template <int EPI, bool LORA, bool I8 = false, bool TM = false>
 static hipError_t launch_epi(const int8_t* Xp, const int8_t* Wp, const float* xs, const float* ws,
-                             const float* bias, void* out, int M, int N, int K, const LoraArgs& la,
-                             hipStream_t st, int nsplit = 1) {
+                             const void* bias, void* out, int M, int N, int K, const LoraArgs& la,
+                             hipStream_t st, int nsplit = 1, int bias_dt = DT_F32) {
     const int Kb = I8 ? K : K / 2;
     if (TM || Kb % P_ROWB == 0) {
         constexpr int WN = CONVROT_PIPE_WN;
@@ -452,12 +455,13 @@ static hipError_t launch_epi(const int8_t* Xp, const int8_t* Wp, const float* xs
         if (e != hipSuccess) return e;
         const int splits = min(nsplit, Kb / P_ROWB);
         hipLaunchKernelGGL((w4a4_gemm_pipe_kernel<EPI, WN, LORA, I8, TM>), dim3(ntiles, splits), dim3(128 * WN),
-                           P_LDS_BYTES, st, Xp, Wp, xs, ws, bias, out, M, N, K, la,
+                           P_LDS_BYTES, st, Xp, Wp, xs, ws, bias, bias_dt, out, M, N, K, la,
                            tile_group_rows((M + P_BM - 1) / P_BM));
     } else if constexpr (!TM) {
         const int splits = min(nsplit, (Kb + ROWB - 1) / ROWB);
         dim3 grid((N + TBN - 1) / TBN, (M + TBM - 1) / TBM, splits), block(NTHR);
-        hipLaunchKernelGGL((w4a4_gemm_kernel<EPI, LORA, I8>), grid, block, 0, st, Xp, Wp, xs, ws, bias, out, M, N, K, la);
+        hipLaunchKernelGGL((w4a4_gemm_kernel<EPI, LORA, I8>), grid, block, 0, st, Xp, Wp, xs, ws,
+                           reinterpret_cast<const float*>(bias), out, M, N, K, la);
     }
     return hipGetLastError();
 }
@@ -466,6 +470,7 @@ hipError_t gemm_launch(const int8_t* Xp, const int8_t* Wp, const float* xs, cons
                        const float* bias, void* out, int M, int N, int K, int epi, hipStream_t st) {
     if (M == 0 || N == 0) return hipSuccess;
     const LoraArgs none{nullptr, nullptr, 0, 0.0f};
+    if (K % 128 == 64) return gemm_p4_launch(Xp, Wp, xs, ws, bias, DT_F32, out, M, N, K, none, epi, st);
     switch (epi) {
         case EPI_F32: return launch_epi<EPI_F32, false>(Xp, Wp, xs, ws, bias, out, M, N, K, none, st);
         case EPI_BF16: return launch_epi<EPI_BF16, false>(Xp, Wp, xs, ws, bias, out, M, N, K, none, st);
@@ -489,16 +494,16 @@ hipError_t gemm_i8_launch(const int8_t* X, const int8_t* W, const float* xs, con
     }
 }
 
-// W8A8 GEMM on I8T operands (K % 64 == 0; rows of A and W padded to 256)
-hipError_t gemm_i8t_launch(const int8_t* X, const int8_t* W, const float* xs, const float* ws,
-                           const float* bias, void* out, int M, int N, int K, int epi, hipStream_t st) {
-    if (M == 0 || N == 0) return hipSuccess;
-    if (K % 64 != 0) return hipErrorInvalidValue;
+// W8A8 GEMM on I8T operands (K % 64 == 0; rows of A and W padded to 256) on the
+// 256 x 256 tiles of large grids; gemm_i8t_launch (gemm_int.hip) chooses.
+hipError_t gemm_i8t_large_launch(const int8_t* X, const int8_t* W, const float* xs, const float* ws, const void* bias,
+                                 int bias_dt, void* out, int M, int N, int K, int epi, hipStream_t st) {
     const LoraArgs none{nullptr, nullptr, 0, 0.0f};
     switch (epi) {
-        case EPI_F32: return launch_epi<EPI_F32, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st);
-        case EPI_BF16: return launch_epi<EPI_BF16, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st);
-        case EPI_ACC: return launch_epi<EPI_ACC, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st);
+        case EPI_F32: return launch_epi<EPI_F32, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st, 1, bias_dt);
+        case EPI_BF16: return launch_epi<EPI_BF16, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st, 1, bias_dt);
+        case EPI_ACC: return launch_epi<EPI_ACC, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st, 1, bias_dt);
+        case EPI_F16: return launch_epi<EPI_F16, false, true, true>(X, W, xs, ws, bias, out, M, N, K, none, st, 1, bias_dt);
         default: return hipErrorInvalidValue;
     }
 }
@@ -588,6 +593,7 @@ hipError_t gemm_lora_launch(const int8_t* Xp, const int8_t* Wp, const float* xs,
                             int M, int N, int K, int epi, hipStream_t st) {
     if (M == 0 || N == 0) return hipSuccess;
     const LoraArgs la{reinterpret_cast<const __bf16*>(t), reinterpret_cast<const __bf16*>(U), R, scale};
+    if (K % 128 == 64) return gemm_p4_launch(Xp, Wp, xs, ws, bias, DT_F32, out, M, N, K, la, epi, st);
     switch (epi) {
         case EPI_F32: return launch_epi<EPI_F32, true>(Xp, Wp, xs, ws, bias, out, M, N, K, la, st);
         case EPI_BF16: return launch_epi<EPI_BF16, true>(Xp, Wp, xs, ws, bias, out, M, N, K, la, st);

@@ -82,12 +82,6 @@ __device__ __forceinline__ void stage_scales(float* sc, const float* __restrict_
     }
 }
 
-__device__ __forceinline__ void stage_scales(float* sc, const float* __restrict__ xs, const float* __restrict__ ws,
-                                             const float* __restrict__ bias, int M, int N, int m0, int n0,
-                                             int tid, int nthreads) {
-    stage_scales(sc, xs, ws, static_cast<const void*>(bias), DT_F32, M, N, m0, n0, tid, nthreads);
-}
-
 // The same staging in two steps: load() issues the global loads into
 // registers at kernel start, ahead of the main loop's first copies, so their
 // latency overlaps the copies' instead of preceding them (stage_scales waits
