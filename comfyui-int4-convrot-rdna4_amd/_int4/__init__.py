@@ -303,6 +303,8 @@ def convrot_w4a4_linear(
             down, up = native._aligned(lora[0]), native._aligned(lora[1])
         native._check_cuda(x2d, w, wsc, b32, down, up)
         x2d = native._aligned(x2d)
+        if x.dtype == torch.float16:
+            epi = native.EPI_F16         # the f32 epilogue rounded to f16 in the kernel, as the cast below would
         if packed:
             out = native.convrot_w4a4_linear_packed(x2d, w, wsc, b32, down, up, 1.0, epi, convrot_groupsize)
         else:
@@ -411,7 +413,8 @@ def convrot_w8a8_linear(
         b = None if b is None else b.contiguous()
         wsc = wscales.to(torch.float32).contiguous()
         native._check_cuda(w8t, wsc, b)
-        epi = native.EPI_F32 if out_dtype == torch.float32 else native.EPI_BF16
+        epi = native.EPI_F16 if x.dtype == torch.float16 else \
+            native.EPI_F32 if out_dtype == torch.float32 else native.EPI_BF16
         out = native.convrot_w8a8_linear_i8t(native._aligned(x2d), native._aligned(w8t), wsc, b, epi,
                                              convrot_groupsize, N)
     else:

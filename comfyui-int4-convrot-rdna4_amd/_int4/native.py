@@ -28,6 +28,8 @@ _DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 _IN_DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 EPI_F32, EPI_BF16, EPI_BF16_EAGER, EPI_ACC = 0, 1, 2, 3
+EPI_F16 = 5    # the one-call linears only
+_OUT_DTYPE = {EPI_F32: torch.float32, EPI_BF16: torch.bfloat16, EPI_BF16_EAGER: torch.bfloat16, EPI_F16: torch.float16}
 
 # cr_abi_version() of the library these signatures describe
 ABI_VERSION = 13
@@ -65,6 +67,8 @@ _SIGNATURES = {
     "cr_convrot_w4a4_linear_bf6_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_bf6_noalloc": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                            + [_vp], _i),
+    "cr_convrot_w4a4_linear_bf6_f16": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 4
+                                       + [_vp, ctypes.c_size_t, _vp], _i),
     "cr_convrot_w8a8_linear_i8t": ([_vp, _i, _vp, _vp, _vp, _i, _vp] + [_i] * 5 + [_vp, ctypes.c_size_t, _vp], _i),
     "cr_convrot_w8a8_linear_i8t_workspace": ([_i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_packed": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
@@ -736,16 +740,17 @@ def convrot_w4a4_linear_bf6(x2d, w6, w_scale, bias, down, up, scale: float, epil
     f32 / bf16 / f16 as stored, or None; down [R, K] / up [N, R] bf16."""
     lib = load_library()
     M, K = x2d.shape
-    odt = {EPI_F32: torch.float32, EPI_BF16: torch.bfloat16, EPI_BF16_EAGER: torch.bfloat16}[epilogue]
-    out = torch.empty((M, N), dtype=odt, device=x2d.device)
+    out = torch.empty((M, N), dtype=_OUT_DTYPE[epilogue], device=x2d.device)
     R = 0 if down is None else down.shape[0]
     nbytes = lib.cr_convrot_w4a4_linear_bf6_workspace(M, N, K, R)
     st = _stream(x2d.device)
     ws = _workspace(x2d.device, st, nbytes)
     bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
-    rc = lib.cr_convrot_w4a4_linear_bf6(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w6), _ptr(w_scale), _ptr(bias),
-                                        bdt, _ptr(down), _ptr(up), R, scale, _ptr(out), epilogue,
-                                        M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    head = (_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w6), _ptr(w_scale), _ptr(bias), bdt, _ptr(down), _ptr(up), R,
+            scale, _ptr(out))
+    tail = (M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    rc = lib.cr_convrot_w4a4_linear_bf6_f16(*head, *tail) if epilogue == EPI_F16 else \
+        lib.cr_convrot_w4a4_linear_bf6(*head, epilogue, *tail)
     if rc != 0:
         raise RuntimeError(f"cr_convrot_w4a4_linear_bf6 failed, hipError={rc}")
     return out
@@ -758,8 +763,7 @@ def convrot_w4a4_linear_packed(x2d, qweight, w_scale, bias, down, up, scale: flo
     lib = load_library()
     M, K = x2d.shape
     N = qweight.shape[0]
-    odt = {EPI_F32: torch.float32, EPI_BF16: torch.bfloat16, EPI_BF16_EAGER: torch.bfloat16}[epilogue]
-    out = torch.empty((M, N), dtype=odt, device=x2d.device)
+    out = torch.empty((M, N), dtype=_OUT_DTYPE[epilogue], device=x2d.device)
     R = 0 if down is None else down.shape[0]
     nbytes = lib.cr_convrot_w4a4_linear_packed_workspace(M, N, K, R)
     st = _stream(x2d.device)
@@ -775,14 +779,14 @@ def convrot_w4a4_linear_packed(x2d, qweight, w_scale, bias, down, up, scale: flo
 
 def convrot_w8a8_linear_i8t(x2d, w8t, w_scale, bias, epilogue: int, convrot_groupsize: int, N: int):
     """The whole W8A8 linear on an I8T weight in one library call; bias [N] f32 /
-    bf16 / f16 as stored, or None; epilogue 0 (f32) or 1 (bf16)."""
+    bf16 / f16 as stored, or None; epilogue 0 (f32), 1 (bf16) or EPI_F16."""
     lib = load_library()
     M, K = x2d.shape
     if w8t.dtype != torch.int8:
         raise ValueError("I8T operands must be int8")
     if w8t.shape[1] != K or w8t.shape[0] != i8t_rows(N):
         raise ValueError(f"I8T operand shape {tuple(w8t.shape)} does not match N={N}, K={K}")
-    out = torch.empty((M, N), dtype=torch.float32 if epilogue == EPI_F32 else torch.bfloat16, device=x2d.device)
+    out = torch.empty((M, N), dtype=_OUT_DTYPE[epilogue], device=x2d.device)
     nbytes = lib.cr_convrot_w8a8_linear_i8t_workspace(M, N, K)
     st = _stream(x2d.device)
     ws = _workspace(x2d.device, st, nbytes)

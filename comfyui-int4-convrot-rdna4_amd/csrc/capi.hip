@@ -377,6 +377,18 @@ static LinPlan int_plan(int bits, int M, int N, int K, int R) {
     return p;
 }
 
+API int cr_convrot_w4a4_linear_bf6_f16(const void* x, int in_dtype, const void* W6, const void* wscale,
+                                       const void* bias, int bias_dtype, const void* D, const void* U, int R,
+                                       float scale, void* out, int M, int N, int K, int G, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+    if (!linear_bf6_args_ok(in_dtype, bias_dtype, D, U, R, convrot::EPI_F32, M, N, K, G)) return -1;
+    if (M == 0 || N == 0) return 0;
+    const LinPlan p = lin_plan(M, N, K, R);
+    if (workspace == nullptr || workspace_bytes < p.total) return -1;
+    return linear_bf6_run(x, in_dtype, W6, wscale, bias, bias_dtype, D, U, R, scale, out, convrot::EPI_F16, M, N, K, G,
+                          p, workspace, stream);
+}
+
 API size_t cr_convrot_w8a8_linear_i8t_workspace(int M, int N, int K) {
     if (M <= 0 || N <= 0 || !i8t_k_ok(K)) return 0;
     return int_plan(8, M, N, K, 0).total;
@@ -386,7 +398,8 @@ API int cr_convrot_w8a8_linear_i8t(const void* x, int in_dtype, const void* W8, 
                                    int bias_dtype, void* out, int epilogue, int M, int N, int K, int G,
                                    void* workspace, size_t workspace_bytes, void* stream) {
     if (!quant_args_ok(in_dtype, M, K, G) || !i8t_k_ok(K) || K > convrot::rotquant_b6_max_k() || N < 0) return -1;
-    if (bias_dtype < 0 || bias_dtype > 2 || (epilogue != 0 && epilogue != 1)) return -1;
+    if (bias_dtype < 0 || bias_dtype > 2) return -1;
+    if (epilogue != convrot::EPI_F32 && epilogue != convrot::EPI_BF16 && epilogue != convrot::EPI_F16) return -1;
     if (M == 0 || N == 0) return 0;
     const LinPlan p = int_plan(8, M, N, K, 0);
     if (workspace == nullptr || workspace_bytes < p.total) return -1;
@@ -411,7 +424,8 @@ API int cr_convrot_w4a4_linear_packed(const void* x, int in_dtype, const void* W
                                       float scale, void* out, int epilogue, int M, int N, int K, int G,
                                       void* workspace, size_t workspace_bytes, void* stream) {
     if (!quant_args_ok(in_dtype, M, K, G) || K % 64 != 0 || N < 0) return -1;
-    if (bias_dtype < 0 || bias_dtype > 2 || epilogue < 0 || epilogue > 2) return -1;
+    if (bias_dtype < 0 || bias_dtype > 2) return -1;
+    if ((epilogue < 0 || epilogue > 2) && epilogue != convrot::EPI_F16) return -1;
     if (R != 0 && (!lora_rank_ok(R) || D == nullptr || U == nullptr || in_dtype == 0)) return -1;
     if (M == 0 || N == 0) return 0;
     const LinPlan p = int_plan(4, M, N, K, R);

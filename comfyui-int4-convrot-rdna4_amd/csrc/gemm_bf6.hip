@@ -270,7 +270,7 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
         const int kc = min(kb, nkb - 1);
         dma16(st + j * 1024, my_src + (size_t)(krev ? nkb - 1 - kc : kc) * B6_CHUNK + j * 1024);
     };
-    // Rank-32 LoRA with a bf16 output: the epilogue's t rows m0 .. m0+255 and U
+    // Rank-32 LoRA with a 16-bit output: the epilogue's t rows m0 .. m0+255 and U
     // rows n0 .. n0+255 (64 bytes each, 32 KB in all, read once per workgroup
     // instead of once per wave) are copied into the ring while the last blocks
     // are multiplied: in phase B of block kb_tu = max(nkb - 2, 0), into that
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     // same stage).  Copy q (0..3) of wave w is 1 KB chunk c = 4 w + q: t rows
     // m0 + 16 c .. for c < 16, U rows n0 + 16 (c - 16) .. above; rows past M / N
     // repeat the last one (they feed only outputs that are never stored).
-    constexpr bool LSTAGE = !SPLIT && LR == 1 && (EPI == EPI_BF16 || EPI == EPI_BF16_EAGER);
+    constexpr bool LSTAGE = !SPLIT && LR == 1 && epi_bytes<EPI> == 2;
     const int kb_tu = nkb >= 2 ? nkb - 2 : 0;
     auto dma_tu = [&](uint32_t st, int q) __attribute__((always_inline)) {
         const int c = wave_u * 4 + q;                            // wave-uniform
@@ -812,6 +812,7 @@ hipError_t gemm_bf6_launch(const void* A6, const void* W6, const float* xs, cons
             case EPI_BF16: return launch_bf6<EPI_BF16, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
             case EPI_BF16_EAGER: return launch_bf6<EPI_BF16_EAGER, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
             case EPI_ACC: return launch_bf6<EPI_ACC, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
+            case EPI_F16: return launch_bf6<EPI_F16, 0>(a, w, xs, ws, bias, bias_dt, out, M, N, K, none, nsplit, part, st);
             default: return hipErrorInvalidValue;
         }
     }
@@ -824,6 +825,7 @@ hipError_t gemm_bf6_launch(const void* A6, const void* W6, const float* xs, cons
             case EPI_F32: return launch_bf6<EPI_F32, LRV>(a, w, xs, ws, bias, bias_dt, out, M, N, K, la, nsplit, part, st);            \
             case EPI_BF16: return launch_bf6<EPI_BF16, LRV>(a, w, xs, ws, bias, bias_dt, out, M, N, K, la, nsplit, part, st);          \
             case EPI_BF16_EAGER: return launch_bf6<EPI_BF16_EAGER, LRV>(a, w, xs, ws, bias, bias_dt, out, M, N, K, la, nsplit, part, st); \
+            case EPI_F16: return launch_bf6<EPI_F16, LRV>(a, w, xs, ws, bias, bias_dt, out, M, N, K, la, nsplit, part, st);          \
             default: return hipErrorInvalidValue;                                                               \
         }
     switch (R / 32) {

@@ -15,6 +15,9 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // EPI_ATOMIC_ACC: the k-split partial of the packed split-K entry point; the
 // exact integer accumulator of the workgroup's k range is added atomically
 // into an int32 [M, N] buffer (integer sums are exact in any order).
+// EPI_F16: the f32 epilogue rounded once to f16, what f16 models store; an f32
+// output with a cast behind it moved the output five times over instead of once
+// (1333 x 2304 -> 6912 on MI355X: the cast 12.5 us).
 enum : int { EPI_F32 = 0, EPI_BF16 = 1, EPI_BF16_EAGER = 2, EPI_ACC = 3, EPI_ATOMIC_ACC = 4,
              EPI_F16 = 5 };
 
@@ -199,14 +202,14 @@ __device__ __forceinline__ void epilogue_tiles(const AccV (&acc)[FMT][FNT], cons
 // LR selects the LoRA term: 0 none; -1 rank la.R read at run time (one
 // dependent t / U load pair per 16 ranks and tile); 1..4 rank 32 * LR known at
 // compile time, loaded in batches of 32 ranks (two t and two U fragments) per
-// tile.  For rank 32 with a bf16 output the t fragments of all the wave's row
+// tile.  For rank 32 with a 16-bit output the t fragments of all the wave's row
 // tiles and the U fragments of its columns are loaded together up front, so
 // the wave waits for them once (a row tile's work is too short to hide the
 // next tile's load: fetching t one row tile ahead cost ~3 us per 256 x 256
 // tile).  The MFMA sequence (16-rank steps in ascending order) is the same in
 // every mode, so are the results.
 //
-// tu_lds (rank 32, bf16 output only): the workgroup tile's t rows tile_m0 ..
+// tu_lds (rank 32, 16-bit output only): the workgroup tile's t rows tile_m0 ..
 // +255 and U rows tile_n0 .. +255 staged in LDS (64 bytes per row, U at
 // +16384), read there instead of from global memory.
 template <int EPI, int FMT, int FNT, int LR, int SCR_BYTES, int ASH = 8, bool HOIST = false, typename AccV>

@@ -261,7 +261,12 @@ int cr_convrot_w4a4_linear_bf6(const void* x, int in_dtype, const void* W6, cons
                                int epilogue, int M, int N, int K, int G, void* workspace, size_t workspace_bytes,
                                void* stream);
 
-/* Workspace bytes of cr_convrot_w4a4_linear_bf6 for this shape and LoRA rank. */
+/* cr_convrot_w4a4_linear_bf6 with epilogue 0's f32 value rounded once to an f16 output. */
+int cr_convrot_w4a4_linear_bf6_f16(const void* x, int in_dtype, const void* W6, const void* wscale, const void* bias,
+                                   int bias_dtype, const void* D, const void* U, int R, float scale, void* out, int M,
+                                   int N, int K, int G, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Workspace bytes of cr_convrot_w4a4_linear_bf6 (and _f16) for this shape and LoRA rank. */
 size_t cr_convrot_w4a4_linear_bf6_workspace(int M, int N, int K, int R);
 
 /*
@@ -342,8 +347,8 @@ int cr_int8_convrot_gemm_i8t(const void* X, const void* W, const void* xscale, c
 /*
  * The whole W8A8 linear in one call: cr_convrot_quant_int8_i8t on x, then the
  * GEMM on W8 (I8T, cr_int8_to_i8t) with the bias read as stored (bias_dtype 0
- * f32, 1 bf16, 2 f16, or NULL) and epilogue 0 (f32) or 1 (bf16); the same bits as
- * those calls.  The codes, scales and split partials live in `workspace` (>= the
+ * f32, 1 bf16, 2 f16, or NULL) and epilogue 0 (f32), 1 (bf16) or 5 (f16: the f32
+ * value rounded once); the same bits as those calls.  The codes, scales and split partials live in `workspace` (>= the
  * _workspace bytes; a new one's first 2048 bytes are zero, every call leaves them
  * so).  No counterpart in the reference's ABI: it serves the per-call sequence of
  * _int4/__init__.py:141-175.
@@ -356,7 +361,7 @@ size_t cr_convrot_w8a8_linear_i8t_workspace(int M, int N, int K);
 /*
  * cr_convrot_w4a4_linear_bf6 on the packed int4 weight Wp [N, K/2] itself, for
  * widths the B6T layout does not hold: K % 64 == 0, K <= cr_max_quant_k(); the
- * same arguments otherwise, the same bits as ck_convrot_quant_int4, cr_lora_down
+ * same arguments otherwise, epilogue 5 (f16) too; the same bits as ck_convrot_quant_int4, cr_lora_down
  * and cr_int4_convrot_gemm_ex / _lora called one by one.
  */
 int cr_convrot_w4a4_linear_packed(const void* x, int in_dtype, const void* Wp, const void* wscale, const void* bias,
