@@ -247,6 +247,13 @@ def convrot_w4a4_linear(
     f16 x the output is the fp32 epilogue rounded once to f16 (the eager f16
     chain, which overflows once |acc| > 65504, is not reproduced).
     """
+    if type(x) is torch.Tensor and x.is_cuda and quant_group_size == _INT4_GROUP_SIZE \
+            and linear_dtype in ("int4", "int8"):
+        y = native.host_module().w4a4(x, qweight, wscales, bias, convrot_groupsize, linear_dtype == "int8", lora,
+                                      qweight_bf6)
+        if y is not None:
+            return y
+    # every form the native host path leaves
     if linear_dtype not in {"int4", "int8"}:
         raise ValueError(f"ConvRot W4A4 linear_dtype must be 'int4' or 'int8', got {linear_dtype!r}")
     if quant_group_size != _INT4_GROUP_SIZE:
@@ -394,6 +401,10 @@ def convrot_w8a8_linear(
     reads ``qweight_i8t`` (from :func:`prepare_convrot_w8a8_weight_i8t`, made
     once at load time; re-laid here when not given): the same codes and
     accumulators, bit-identical outputs."""
+    if type(x) is torch.Tensor and x.is_cuda:
+        y = native.host_module().w8a8(x, qweight, wscales, bias, convrot_groupsize, qweight_i8t)
+        if y is not None:
+            return y
     if x.shape[-1] != qweight.shape[-1]:
         raise ValueError(f"Input K={x.shape[-1]} does not match qweight K={qweight.shape[-1]}")
     if x.shape[-1] % convrot_groupsize != 0:

@@ -3,14 +3,17 @@ JIT ``_int4/build.py``, which compiled for whatever arch the GPU reported).
 
 ``build()`` runs hipcc for gfx950 only: every source is compiled to an object
 in parallel (``_build/`` next to this file), then the objects are linked into
-``libconvrot_gfx950.so`` next to this file.  The library is loaded by
+``libconvrot_gfx950.so`` next to this file, and the host module ``_host.so``
+(csrc/host.cpp) against it.  Both are loaded by
 ``native.py``; nothing builds at import or at first use.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -25,18 +28,22 @@ def lib_path() -> str:
     return os.path.join(_HERE, "libconvrot_gfx950.so")
 
 
+def host_path() -> str:
+    return os.path.join(_HERE, "_host.so")
+
+
 def sources() -> list[str]:
     return [os.path.join(_CSRC, s) for s in SOURCES]
 
 
 def _deps() -> list[str]:
-    return sources() + [os.path.join(_CSRC, h) for h in HEADERS] + [
+    return sources() + [os.path.join(_CSRC, h) for h in HEADERS + ("host.cpp",)] + [
         os.path.join(os.path.dirname(_PKG), "include", "convrot_mi355x.h")]
 
 
 def is_stale() -> bool:
     out = lib_path()
-    if not os.path.exists(out):
+    if not os.path.exists(out) or not os.path.exists(host_path()):
         return True
     t = os.path.getmtime(out)
     return any(os.path.getmtime(d) > t for d in _deps() if os.path.exists(d))
@@ -75,20 +82,52 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _torch_dir() -> str:
+    return os.path.dirname(importlib.util.find_spec("torch").origin)
+
+
+def _run(cmd: list[str], out: str, what: str) -> None:
+    cp = subprocess.run([*cmd, "-o", out + ".tmp"], capture_output=True, text=True)
+    if cp.returncode != 0 or not os.path.exists(out + ".tmp"):
+        raise RuntimeError(f"{what} failed:\n{cp.stderr}")
+    os.replace(out + ".tmp", out)
+
+
+def _compile_host() -> str:
+    """csrc/host.cpp (host code only) against torch's headers."""
+    inc = os.path.join(_torch_dir(), "include")
+    rocm = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "include")
+    obj = os.path.join(_obj_dir(), "host.cpp.o")
+    _run([_hipcc(), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+          "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+          "-isystem", sysconfig.get_paths()["include"], "-isystem", rocm, "-x", "c++", "-c",
+          os.path.join(_CSRC, "host.cpp")], obj, "hipcc on host.cpp")
+    return obj
+
+
+def _link_host(obj: str, lib: str) -> None:
+    """The CPython module, bound to the kernel library next to it."""
+    _run([_hipcc(), "-shared", "-fPIC", "-Wl,--as-needed", obj, "-L" + os.path.join(_torch_dir(), "lib"), "-ltorch_python", "-ltorch_cpu",
+          "-lc10", "-lc10_hip", "-L" + os.path.dirname(lib), "-l:" + os.path.basename(lib), "-Wl,-rpath,$ORIGIN"],
+         host_path(), "linking the host module")
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> str:
     out = lib_path()
     tmp = out + ".tmp"
     srcs = sources()
     if verbose:
         print("building:", " ".join([_hipcc(), *CFLAGS, "-c", "<src>"]), "for", ", ".join(SOURCES))
-    n = jobs or min(len(srcs), max(1, (os.cpu_count() or 4)))
+    n = jobs or min(len(srcs) + 1, max(1, (os.cpu_count() or 4)))
     with ThreadPoolExecutor(max_workers=n) as ex:
+        host = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
     cp = subprocess.run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp],
                         capture_output=True, text=True)
     if cp.returncode != 0 or not os.path.exists(tmp):
         raise RuntimeError(f"hipcc link failed:\n{cp.stderr}")
     os.replace(tmp, out)
+    _link_host(host.result(), out)
     return out
 
 

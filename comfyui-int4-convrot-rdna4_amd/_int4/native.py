@@ -13,6 +13,8 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -70,6 +72,8 @@ _SIGNATURES = {
     "cr_convrot_w4a4_linear_bf6_f16": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 4
                                        + [_vp, ctypes.c_size_t, _vp], _i),
     "cr_convrot_w8a8_linear_i8t": ([_vp, _i, _vp, _vp, _vp, _i, _vp] + [_i] * 5 + [_vp, ctypes.c_size_t, _vp], _i),
+    "cr_convrot_w4a4_linear_bf6_split": ([_i, _i, _i], _i),
+    "cr_convrot_w8a8_linear_i8t_split": ([_i, _i, _i], _i),
     "cr_convrot_w8a8_linear_i8t_workspace": ([_i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_packed": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                       + [_vp, ctypes.c_size_t, _vp], _i),
@@ -110,6 +114,27 @@ def load_library():
             fn.restype = res
         _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host_module():
+    """The native host path of the linears (csrc/host.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load_library()                       # checks the ABI version of the library it calls
+        with _lock:
+            if _host is None:
+                path = _build.host_path()
+                if not os.path.exists(path):
+                    raise RuntimeError(f"{os.path.basename(path)} is not built; run the package's _int4/build.py first")
+                loader = importlib.machinery.ExtensionFileLoader("_host", path)
+                spec = importlib.util.spec_from_file_location("_host", path, loader=loader)
+                mod = importlib.util.module_from_spec(spec)
+                loader.exec_module(mod)
+                _host = mod
+    return _host
 
 
 def exported_symbols() -> list[str]:

@@ -304,6 +304,10 @@ API size_t cr_convrot_w4a4_linear_bf6_workspace(int M, int N, int K, int R) {
     return lin_plan(M, N, K, R).total;
 }
 
+API int cr_convrot_w4a4_linear_bf6_split(int M, int N, int K) {
+    return M > 0 && N > 0 && bf6_k_ok(K) && lin_plan(M, N, K, 0).nsplit > 1;
+}
+
 static int linear_bf6_args_ok(int in_dtype, int bias_dtype, const void* D, const void* U, int R, int epilogue,
                               int M, int N, int K, int G) {
     if (!quant_args_ok(in_dtype, M, K, G) || !bf6_k_ok(K) || K > convrot::rotquant_b6_max_k() || N < 0) return 0;
@@ -392,6 +396,10 @@ API int cr_convrot_w4a4_linear_bf6_f16(const void* x, int in_dtype, const void* 
 API size_t cr_convrot_w8a8_linear_i8t_workspace(int M, int N, int K) {
     if (M <= 0 || N <= 0 || !i8t_k_ok(K)) return 0;
     return int_plan(8, M, N, K, 0).total;
+}
+
+API int cr_convrot_w8a8_linear_i8t_split(int M, int N, int K) {
+    return M > 0 && N > 0 && i8t_k_ok(K) && int_plan(8, M, N, K, 0).nsplit > 1;
 }
 
 API int cr_convrot_w8a8_linear_i8t(const void* x, int in_dtype, const void* W8, const void* wscale, const void* bias,

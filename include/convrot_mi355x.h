@@ -269,6 +269,11 @@ int cr_convrot_w4a4_linear_bf6_f16(const void* x, int in_dtype, const void* W6, 
 /* Workspace bytes of cr_convrot_w4a4_linear_bf6 (and _f16) for this shape and LoRA rank. */
 size_t cr_convrot_w4a4_linear_bf6_workspace(int M, int N, int K, int R);
 
+/* 1 when the linear's GEMM splits k over workgroups, so that its workspace's
+ * counters (the first 2048 bytes) have to be zero; 0: any workspace will do. */
+int cr_convrot_w4a4_linear_bf6_split(int M, int N, int K);
+int cr_convrot_w8a8_linear_i8t_split(int M, int N, int K);
+
 /*
  * cr_convrot_w4a4_linear_bf6 without the workspace argument: the library
  * allocates nothing during the call (no hipMalloc, no allocating library
