@@ -116,4 +116,11 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
+// The same for f16 (past the range to infinity).
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+    const f16x2_t h = __builtin_convertvector((f32x2_t){a, b}, f16x2_t);
+    return __builtin_bit_cast(uint32_t, h);
+}
+
 }  // namespace convrot

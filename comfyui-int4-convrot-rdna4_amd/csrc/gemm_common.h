@@ -29,7 +29,7 @@ template <int EPI> constexpr int epi_bytes = EPI == EPI_BF16 || EPI == EPI_BF16_
 template <int EPI>
 __device__ __forceinline__ uint32_t pack_out2(float a, float b) {
     if constexpr (EPI == EPI_F16)
-        return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
+        return pack_f16x2(a, b);
     else
         return pack_bf16x2(a, b);
 }

@@ -43,7 +43,14 @@
 // So any approximation P of xr/s with relative error below that distance has
 // RNE_DT(P) == RNE_DT(xr/s) == RNE_DT(fl32(xr/s)):
 //   bf16: P = fl32(xr * fl32(1/s)), error <= 2^-23 < 2^-17;
-//   f16:  P = fl32(fl64(xr * fl64(1/s))), error <= 2^-24 + 2^-52 < 2^-23.
+//   f16:  P = t + (xr - s t) r with t = fl32(xr r), r = fl32(1/s) after a Newton
+//         step, both steps fma: the residual is exact but for its own rounding,
+//         so P is within 2^-24 (1 + 2^-20) < 2^-23 (the kernel for stochastic
+//         rounding: fl32(fl64(xr * fl64(1/s))), error <= 2^-24 + 2^-52).  With
+//         the rounding to f16 taken from the jammed floats as for bf16, two values
+//         a conversion, f16 runs 25.4 VALU instructions per element instead of
+//         30.5: packed int4, 12288 x 3072 35.3 -> 29.7 us, B6T 4608 x 3072 17.2 ->
+//         14.6 (MI355X, graph replays).
 // f32 uses the IEEE fp32 division directly.
 
 #include "b6t_layout.h"
@@ -344,18 +351,6 @@ template <int DT> struct Held { uint32_t w[8]; };
 template <> struct Held<DT_F32> { float f[16]; };
 
 template <int DT>
-__device__ __forceinline__ void hold(Held<DT>& h, int i, float a, float b) {   // values i, i+1
-    if constexpr (DT == DT_F32) {
-        h.f[i] = a; h.f[i + 1] = b;
-    } else if constexpr (DT == DT_BF16) {
-        h.w[i >> 1] = (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
-    } else {
-        h.w[i >> 1] = (uint32_t)__half_as_ushort(__float2half_rn(a)) |
-                      ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
-    }
-}
-
-template <int DT>
 __device__ __forceinline__ float held(const Held<DT>& h, int i) {
     if constexpr (DT == DT_F32) return h.f[i];
     else if constexpr (DT == DT_BF16) return (i & 1) ? bf16hi_to_f32(h.w[i >> 1]) : bf16lo_to_f32(h.w[i >> 1]);
@@ -446,16 +441,15 @@ template <int DT>
 __device__ __forceinline__ void hold_chunk(const double (&v)[16], Held<DT>& h, float& lmax) {
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
-        if constexpr (DT == DT_BF16) {
+        if constexpr (DT != DT_F32) {
             // lmax gathers jammed values: its RNE is the max of the rounded values
             const float f0 = jam_to_f32(v[i]), f1 = jam_to_f32(v[i + 1]);
-            h.w[i >> 1] = pack_bf16x2(f0, f1);
+            h.w[i >> 1] = DT == DT_BF16 ? pack_bf16x2(f0, f1) : pack_f16x2(f0, f1);
             lmax = absmax3(lmax, f0, f1);
         } else {
-            const float r0 = round_f64_to_dt<DT>(v[i]);
-            const float r1 = round_f64_to_dt<DT>(v[i + 1]);
-            hold<DT>(h, i, r0, r1);
-            lmax = absmax3(lmax, r0, r1);
+            h.f[i] = (float)v[i];
+            h.f[i + 1] = (float)v[i + 1];
+            lmax = absmax3(lmax, h.f[i], h.f[i + 1]);
         }
     }
 }
@@ -630,7 +624,14 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(4, 5)
         // 2^-22 of xr / s, inside the 2^-17 the quotient keeps from every bf16
         // midpoint (file header)
         const float rinv32 = __builtin_amdgcn_rcpf(s);
-        const double rinv = 1.0 / (double)s;
+        // f16: reciprocal, residual factor and residual reciprocal of the quotient
+        // (file header).  s = 0 (a below half the smallest f16 times QMAX, or a row of
+        // zeros): every nonzero value goes past the clamp and zeros stay 0, as x / 0 did;
+        // s = inf: finite values give 0 and infinities NaN (code 0).  In fp32: three
+        // operations an element against fp64's conversion, product and conversion.
+        const bool regular = s > 0.0f && s < __builtin_inff();
+        const float rc = regular ? __builtin_fmaf(__builtin_fmaf(-s, rinv32, 1.0f), rinv32, rinv32) : s > 0.0f ? 0.0f : 3e38f;
+        const float rneg = regular ? -s : 0.0f, rres = regular ? rc : 0.0f;
         // B6T: the codes of flush f (after passes 2f, 2f+1) stay in registers
         // until every flush of the row is converted, then all are stored: a
         // store issued mid-loop would hold back the next flush, whose registers
@@ -681,10 +682,15 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(4, 5)
                     for (int h = 0; h < 2; ++h) {
                         const float xv = held<DT>(hv[p], i + h);
                         float z;
-                        if constexpr (DT == DT_F32) z = xv / s;
-                        else z = round_to_dt<DT>((float)((double)xv * rinv));
-                        if constexpr (DT == DT_F16) z = (z == z) ? z : 0.0f;
-                        zz[h] = fminf(fmaxf(z, -QMAX), QMAX);
+                        if constexpr (DT == DT_F32) {
+                            z = xv / s;
+                        } else {
+                            const float t = xv * rc;
+                            z = round_to_dt<DT>(__builtin_fmaf(__builtin_fmaf(rneg, t, xv), rres, t));
+                            z = (z == z) ? z : 0.0f;
+                        }
+                        // f16: no NaN is left, one v_med3
+                        zz[h] = DT == DT_F16 ? __builtin_amdgcn_fmed3f(z, -QMAX, QMAX) : fminf(fmaxf(z, -QMAX), QMAX);
                     }
                     z0 = zz[0];
                     z1 = zz[1];
