@@ -860,6 +860,20 @@ static hipError_t rq_row_launch(const void* x, int8_t* q, float* s, int M, int K
         if (np <= 24) return rq_wide_launch<DT, G, 3, OUT, LR>(x, q, s, M, K, 8, st, ls);
         return rq_wide_launch<DT, G, 2, OUT, LR>(x, q, s, M, K, 16, st, ls);
     }
+    // Few rows of 5 to 12 passes: one pass per wave (or two, five waves to a row),
+    // on the 16-wave instance, while every row's workgroup is resident at once (16
+    // waves per CU): a row is a serial chain of loads, rotations and the absmax,
+    // which nothing else hides on such a grid.  Measured on MI355X (graph replays,
+    // bf16 -> I8T, us, 4 waves and one pass per wave): 1 x 5120 3.6 / 3.2, 512 x
+    // 5120 5.1 / 4.5, 256 x 8192 4.4 / 3.9, 256 x 9216 5.2 / 4.3, 256 x 12288 5.6 /
+    // 4.5; two passes on five waves: 512 x 9216 6.7 / 5.9, 768 x 9216 8.4 / 7.4.  At
+    // 512 x 12288 six waves of two passes took 7.5 against 7.2, so rows of 11 and 12
+    // passes keep four waves there.
+    if (np > kRowMaxWaves) {
+        const int w2 = (np + 1) / 2;
+        if (M <= 256 * (16 / np)) return rq_wide_launch<DT, G, 1, OUT, LR>(x, q, s, M, K, np, st, ls);
+        if (np > 8 && w2 <= 5 && M <= 768) return rq_wide_launch<DT, G, 2, OUT, LR>(x, q, s, M, K, w2, st, ls);
+    }
     int W, P;
     if (np <= 2 * kRowMaxWaves) {
         P = np <= kRowMaxWaves ? np : (np % 3 != 0 ? 2 : 3);

@@ -1,9 +1,36 @@
-"""The f16 quotient of rotate+quant at the ends of its range against the eager
+"""Launch shapes of rotate+quant on few long rows against the many-row launch
+and the oracle, and the f16 quotient at the ends of its range against the eager
 arithmetic."""
+import numpy as np
 import pytest
 import torch
 
+from inputs import outlier_activations
+
 pytestmark = pytest.mark.gpu
+
+
+# the last row count of each launch shape and the next: 5, 7, 8, 9, 10, 11 and 12 passes of 1024
+@pytest.mark.parametrize("K,Ms", [(5120, (1, 768, 769)), (6400, (512, 513)), (8192, (512, 513)), (8448, (256, 257, 768, 769)),
+                                  (10240, (256, 768)), (10496, (256, 257)), (12288, (1, 256, 257))])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_few_rows(native, oracle, gpu, K, Ms, dt):
+    print(f"few rows K={K} {dt}", flush=True)
+    x = outlier_activations(1100, K, seed=K).to(dt).cuda()
+    q, s = native.convrot_quant_int4(x, 256)
+    q8, s8 = native.convrot_quant_int8(x, 256)
+    code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dt]
+    h = x[:3].cpu()
+    raw = h.numpy() if dt == torch.float32 else h.view(torch.int16).numpy().view(np.uint16)
+    eq, es, _ = oracle.rotquant(raw, code, 256)
+    assert np.array_equal(q[:3].cpu().numpy(), eq) and np.array_equal(s[:3].cpu().numpy(), es)
+    for M in Ms:
+        qm, sm = native.convrot_quant_int4(x[:M], 256)
+        assert torch.equal(qm, q[:M]) and torch.equal(sm, s[:M]), M
+        a6, s6 = native.convrot_quant_bf6(x[:M], 256)
+        assert torch.equal(native.bf6_to_int4(a6, M, K), q[:M]) and torch.equal(s6, s[:M]), M
+        at, st = native.convrot_quant_int8_i8t(x[:M], 256)
+        assert torch.equal(native.i8t_to_int8(at, M), q8[:M]) and torch.equal(st, s8[:M]), M
 
 
 def h4():
