@@ -150,6 +150,23 @@ __device__ __forceinline__ v8i bf6_operand_odd(v4u q, v4u p) {
     return (v8i){(int)q.z, (int)q.w, (int)p.x, (int)p.y, (int)p.z, (int)p.w, 0, 0};
 }
 
+// The large tile of WN waves along N: 256 x 256 (WN 4), or 256 x 192 (WN 3, six
+// waves, seven copies each, B in units of 64 rows as in the small-tile kernel).
+constexpr int B6S_UNIT = 6144;                                  // 64 rows of a chunk: P 4 KB + Q 2 KB
+constexpr int B6S_UNIT_Q = 4096;                                // Q part inside a unit
+template <int WN>
+struct B6Large {
+    static constexpr int BN = 64 * WN;
+    static constexpr int STAGE = B6_CHUNK + WN * B6S_UNIT;
+    static constexpr int RING = B6_STAGES * STAGE;
+    static constexpr int LDS = RING + EPI_SCALE_FLOATS * 4;
+    static constexpr int LOADS = STAGE / 1024 / (2 * WN);
+    static constexpr int TU = (256 + BN) / 16 / (2 * WN) + (WN == 3);   // 1 KB copies of t / U per wave, rounded up
+    static_assert(WN == 3 || WN == 4, "tile");
+};
+static_assert(B6Large<4>::STAGE == B6_STAGE_BYTES && B6Large<4>::LDS == B6_LDS_BYTES && B6Large<4>::LOADS == B6_LOADS,
+              "256 x 256");
+
 // SPLIT: split-K partial kernel.  Workgroup b takes tile b % T and the 128-k
 // blocks [s nkb / S, (s + 1) nkb / S) of split s = b / T (T tiles, S splits),
 // and stores its raw accumulators (exact integers in fp32) in the workspace in
@@ -157,8 +174,8 @@ __device__ __forceinline__ v8i bf6_operand_odd(v4u q, v4u p) {
 // (q * 64 + lane) * 4 + e] = acc[q / 8][(q / 4) % 2][4 (q % 4) + e].  The
 // scales, the epilogue and the LoRA term run once per output, in the reduce
 // kernel below.
-template <int EPI, int LR, bool SPLIT>
-__global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
+template <int EPI, int LR, bool SPLIT, int WN = 4>
+__global__ __launch_bounds__(128 * WN) void w4a4_gemm_bf6_kernel(
         const uint8_t* __restrict__ A6, const uint8_t* __restrict__ W6,
         const float* __restrict__ xs, const float* __restrict__ ws, const void* __restrict__ bias, int bias_dt,
         void* __restrict__ out, int M, int N, int K, LoraArgs lora, int gm, int nsplit,
@@ -168,8 +185,10 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int wm = wave >> 2, wn = wave & 3;
-    const int tiles_m = (M + B6_BM - 1) / B6_BM, tiles_n = (N + B6_BN - 1) / B6_BN;
+    using S = B6Large<WN>;
+    static_assert(!SPLIT || WN == 4, "the split kernel runs 256 x 256 tiles");
+    const int wm = wave / WN, wn = wave % WN;
+    const int tiles_m = (M + B6_BM - 1) / B6_BM, tiles_n = (N + S::BN - 1) / S::BN;
     const int nkb_all = K / 128;
     int tm, tn, kb0 = 0, nkb = nkb_all, split = 0, tile = 0;
     if constexpr (SPLIT) {
@@ -184,9 +203,9 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
         tile_of_block(blockIdx.x, tiles_m, tiles_n, gm, tm, tn);
     }
     const int m0 = tm * B6_BM;
-    const int n0 = tn * B6_BN;
+    const int n0 = tn * S::BN;
 
-    float* sc = reinterpret_cast<float*>(lds6 + B6_RING_BYTES);
+    float* sc = reinterpret_cast<float*>(lds6 + S::RING);
     ScaleRegs scr;                                            // staged in LDS after the main loop
     if constexpr (!SPLIT) scr.load(xs, ws, bias, bias_dt, M, N, m0, n0, tid);
 
@@ -196,6 +215,18 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
                                            : W6 + (size_t)tn * nkb_all * B6_CHUNK) + (size_t)kb0 * B6_CHUNK;
     const uint8_t* my_src = my_chunks + (wave_u & 3) * (B6_LOADS * 1024) + lane * 16;
     const uint32_t my_lds = (uint32_t)(uintptr_t)lds6 + wave_u * (B6_LOADS * 1024);
+    // WN = 3: copies 0..3 of a wave are KB 4 w .. 4 w + 3 of the A chunk, copies
+    // 4..6 half of 64-row unit w / 2 of B (its P KB 0, 1, 2 or its P KB 3 and Q).
+    // Units past the padded rows of B repeat the last one.
+    const uint8_t *a_src = nullptr, *b_src[3] = {nullptr, nullptr, nullptr};
+    if constexpr (WN == 3) {
+        a_src = A6 + (size_t)tm * nkb_all * B6_CHUNK + wave_u * 4096;
+        const int gu = min((n0 >> 6) + (wave_u >> 1), ((N + 255) >> 8) * 4 - 1), hu = gu & 3;
+        const uint8_t* unit = W6 + (size_t)(gu >> 2) * nkb_all * B6_CHUNK;
+        b_src[0] = unit + hu * 4096 + (wave_u & 1) * 3072;
+        b_src[1] = wave_u & 1 ? unit + B6_QOFF + hu * 2048 : unit + hu * 4096 + 1024;
+        b_src[2] = b_src[1] + 1024;
+    }
     v16f acc[4][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -220,8 +251,13 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
             const int g = 2 * s2 + fhalf;
             offPa[s2] = b6_p_off(ra, g);
             offQa[s2] = b6_q_off(ra, g);
-            offPb[s2] = B6_CHUNK + b6_p_off(rb, g);
-            offQb[s2] = B6_CHUNK + b6_q_off(rb, g);
+            if constexpr (WN == 4) {
+                offPb[s2] = B6_CHUNK + b6_p_off(rb, g);
+                offQb[s2] = B6_CHUNK + b6_q_off(rb, g);
+            } else {                                          // units of [P 4 KB][Q 2 KB]
+                offPb[s2] = B6_CHUNK + wn * B6S_UNIT + b6_p_off(frow, g);
+                offQb[s2] = B6_CHUNK + wn * B6S_UNIT + B6S_UNIT_Q + b6_q_off(frow, g) - B6_QOFF;
+            }
         }
     }
     // Fragments of one k step: P pieces of the 4 A and 2 B row tiles, and the 16-byte
@@ -266,9 +302,16 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     // 85.6 -> 84.7 us, mlp_up 114.0 -> 111.3 us, one-round shapes unchanged.
     const bool krev = !SPLIT && ((blockIdx.x >> 3) / 32 & 1);
     auto dma_one = [&](int kb, int j) __attribute__((always_inline)) {
-        const uint32_t st = my_lds + (kb % B6_STAGES) * B6_STAGE_BYTES;
         const int kc = min(kb, nkb - 1);
-        dma16(st + j * 1024, my_src + (size_t)(krev ? nkb - 1 - kc : kc) * B6_CHUNK + j * 1024);
+        const size_t ko = (size_t)(krev ? nkb - 1 - kc : kc) * B6_CHUNK;
+        if constexpr (WN == 4) {
+            const uint32_t st = my_lds + (kb % B6_STAGES) * S::STAGE;
+            dma16(st + j * 1024, my_src + ko + j * 1024);
+        } else {
+            const uint32_t st = (uint32_t)(uintptr_t)lds6 + (kb % B6_STAGES) * S::STAGE;
+            if (j < 4) dma16_sv(st + wave_u * 4096 + j * 1024, a_src + ko + j * 1024, lane * 16);
+            else dma16_sv(st + B6_CHUNK + wave_u * 3072 + (j - 4) * 1024, b_src[j - 4] + ko, lane * 16);
+        }
     };
     // Rank-32 LoRA with a 16-bit output: the epilogue's t rows m0 .. m0+255 and U
     // rows n0 .. n0+255 (64 bytes each, 32 KB in all, read once per workgroup
@@ -276,13 +319,13 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     // are multiplied: in phase B of block kb_tu = max(nkb - 2, 0), into that
     // block's stage, in place of the past-the-end copies that would have gone
     // there (the last block's phase A skips its own past-the-end copy into the
-    // same stage).  Copy q (0..3) of wave w is 1 KB chunk c = 4 w + q: t rows
+    // same stage).  Copy q of wave w is 1 KB chunk c = TU w + q (TU 4; 5 of 256 x 192): t rows
     // m0 + 16 c .. for c < 16, U rows n0 + 16 (c - 16) .. above; rows past M / N
     // repeat the last one (they feed only outputs that are never stored).
     constexpr bool LSTAGE = !SPLIT && LR == 1 && epi_bytes<EPI> == 2;
     const int kb_tu = nkb >= 2 ? nkb - 2 : 0;
     auto dma_tu = [&](uint32_t st, int q) __attribute__((always_inline)) {
-        const int c = wave_u * 4 + q;                            // wave-uniform
+        const int c = min(wave_u * S::TU + q, 15 + S::BN / 16);   // wave-uniform; past the last chunk: again
         const bool is_t = c < 16;
         const int r0 = is_t ? m0 + c * 16 : n0 + (c - 16) * 16;   // may lie past M / N (edge tiles)
         const int last = (is_t ? M : N) - 1;
@@ -306,13 +349,13 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     // a row); sched_barrier(0) pins every slot.
     Frags F0, F1;
 #pragma unroll
-    for (int j = 0; j < B6_LOADS; ++j) dma_one(0, j);
+    for (int j = 0; j < S::LOADS; ++j) dma_one(0, j);
 #pragma unroll
-    for (int j = 0; j < B6_LOADS; ++j) dma_one(1, j);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(B6_LOADS));          // block 0 landed, block 1 in flight
+    for (int j = 0; j < S::LOADS; ++j) dma_one(1, j);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(S::LOADS));          // block 0 landed, block 1 in flight
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < B6_LOADS / 2; ++j) dma_one(2, j);    // first half; the second in phase A of block 0
+    for (int j = 0; j < S::LOADS / 2; ++j) dma_one(2, j);    // first half; the second in phase A of block 0
 #pragma unroll
     for (int r = 0; r < 9; ++r) read_one(0, 0, r, F0);
     uint32_t st_cur = 0;                                      // stage of block kb
@@ -323,19 +366,20 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     // extra branches or registers.
     auto block = [&](int kb, auto mode_c) __attribute__((always_inline)) {
         constexpr int MODE = decltype(mode_c)::value;
-        const uint32_t st_nxt = st_cur == (B6_STAGES - 1) * B6_STAGE_BYTES ? 0u : st_cur + B6_STAGE_BYTES;
+        const uint32_t st_nxt = st_cur == (B6_STAGES - 1) * S::STAGE ? 0u : st_cur + S::STAGE;
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             mfma_one(F0, t);
             __builtin_amdgcn_sched_barrier(0);
-            if (MODE != 2 && (t == 2 || t == 4 || t == 6)) dma_one(kb + 2, B6_LOADS / 2 + (t - 2) / 2);
+            if (WN == 3 && MODE != 2 && t == 1) dma_one(kb + 2, 3);
+            if (MODE != 2 && (t == 2 || t == 4 || t == 6)) dma_one(kb + 2, S::LOADS - 3 + (t - 2) / 2);
             reads_after(t, st_cur, 1, F1);
             __builtin_amdgcn_sched_barrier(0);
         }
         // this wave's copies of block kb+1 landed (the six of block kb+2 may be in
         // flight) and its reads of block kb done: after the barrier block kb's
         // stage is free
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(B6_LOADS) & 0xc07f);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(S::LOADS) & 0xc07f);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -346,6 +390,7 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
                 if (MODE == 1) {
                     dma_tu(st_cur, t == 2 ? 0 : t == 4 ? 1 : 2);
                     if (t == 6) dma_tu(st_cur, 3);
+                    if (t == 6 && S::TU == 5) dma_tu(st_cur, 4);
                 } else {
                     dma_one(kb + 3, (t - 2) / 2);
                 }
@@ -381,15 +426,15 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
     int em0 = m0, en0 = n0, elane = lane;
     asm volatile("" : "+s"(M), "+s"(N), "+v"(em0), "+v"(en0), "+v"(elane));
     if constexpr (LSTAGE) {
-        // t / U sit in the first 32 KB of stage kb_tu % 3; the waves' output
-        // scratch (12 KB each) fills the other two stages
+        // t / U sit in the first 32 KB (28 of 256 x 192) of stage kb_tu % 3; the
+        // waves' output scratch fills the other two stages
         const int tu = kb_tu % B6_STAGES;
-        constexpr int SCR = 2 * B6_STAGE_BYTES / (B6_THREADS / 64);
-        uint8_t* scr = lds6 + ((tu + 1 + (wave >> 2)) % B6_STAGES) * B6_STAGE_BYTES + (wave & 3) * SCR;
+        constexpr int SCR = S::STAGE / WN;
+        uint8_t* scr = lds6 + ((tu + 1 + wave / WN) % B6_STAGES) * S::STAGE + wave % WN * SCR;
         epilogue_lds<EPI, 4, 2, LR, SCR>(acc, sc, out, M, N, em0, en0, em0 + wm * 128, en0 + wn * 64, elane, lora,
-                                         scr, lds6 + tu * B6_STAGE_BYTES);
+                                         scr, lds6 + tu * S::STAGE);
     } else {
-        constexpr int SCR = B6_RING_BYTES / (B6_THREADS / 64);
+        constexpr int SCR = S::RING / (2 * WN);
         epilogue_lds<EPI, 4, 2, LR, SCR>(acc, sc, out, M, N, em0, en0, em0 + wm * 128,
                                          en0 + wn * 64, elane, lora, lds6 + wave * SCR);
     }
@@ -430,8 +475,6 @@ __global__ __launch_bounds__(B6_THREADS) void w4a4_gemm_bf6_kernel(
 // the grid.  The counters (one per tile, at most 512) must be zero when a
 // workspace is first used; every call leaves them zero.
 // ---------------------------------------------------------------------------
-constexpr int B6S_UNIT = 6144;                                  // 64 rows of a chunk: P 4 KB + Q 2 KB
-constexpr int B6S_UNIT_Q = 4096;                                // Q part inside a unit
 constexpr int B6S_STAGES = 3;                                   // 128 x 128: 4 and 6 measured no faster
 constexpr int B6S_MAX_SPLIT_TILES = 512;                        // split counters per workspace
 constexpr int B6S_BM = 128, B6S_BN = 128;                       // the quarter tile
@@ -693,6 +736,7 @@ __global__ __launch_bounds__(64 * B6R_WAVES) void w4a4_bf6_splitk_reduce_kernel(
 
 bool gemm_bf6_small_tiles(int M, int N, int K);
 int gemm_bf6_small_shape(int M, int N, int K, int nsplit);
+int gemm_bf6_large_shape(int M, int N, int K);
 void gemm_bf6_direct_tile(int M, int N, int K, int* bm, int* bn);
 hipError_t gemm_bf6_direct_launch(const uint8_t* A, const uint8_t* B, const float* xs, const float* ws,
                                   const void* bias, int bias_dt, void* out, int M, int N, int K, const LoraArgs& la,
@@ -758,6 +802,16 @@ static hipError_t launch_bf6(const uint8_t* A6, const uint8_t* W6, const float* 
     }
     const int tiles_m = (M + B6_BM - 1) / B6_BM;
     const int ntiles = tiles_m * ((N + B6_BN - 1) / B6_BN);
+    if (nsplit <= 1 && gemm_bf6_large_shape(M, N, K) == 192) {
+        static std::atomic<bool> attr_192[kMaxDev];
+        e = lds_limit_once(attr_192, dev, reinterpret_cast<const void*>(&w4a4_gemm_bf6_kernel<EPI, LR, false, 3>),
+                           B6Large<3>::LDS);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((w4a4_gemm_bf6_kernel<EPI, LR, false, 3>), dim3(tiles_m * ((N + 191) / 192)), dim3(384),
+                           B6Large<3>::LDS, st, A6, W6, xs, ws, bias, bias_dt, out, M, N, K, la,
+                           tile_group_rows(tiles_m), 1, nullptr);
+        return hipGetLastError();
+    }
     if (nsplit <= 1) {
         e = lds_limit_once(attr_set, dev, reinterpret_cast<const void*>(&w4a4_gemm_bf6_kernel<EPI, LR, false>),
                            B6_LDS_BYTES);
@@ -877,12 +931,35 @@ int gemm_bf6_small_shape(int M, int N, int K, int nsplit) {
     return t128 > 256 && t192 <= 256 ? SMALL_128x192 : SMALL_128x128;
 }
 
+// Width of the large tile of an unsplit launch: 192 when the 256 x 192 tiles take
+// no more rounds of the 256 CUs than the 256 x 256 ones, 256 otherwise.  A round
+// costs what one workgroup copies (42 KB a block against 48) and its prologue and
+// epilogue; the narrower tile copies 17% more per output, which shows only in
+// extra rounds.  Measured on MI355X (graph replays, uniform codes, bf16 out, us, 256 x 256 / 256 x
+// 192, tiles in brackets): 4096 x 12288 -> 3072 (192 / 256) 90.5 / 85.6; 1333 x
+// 2304 -> 6912 (162 / 216) 20.3 / 19.4; 3072 x 3072 -> 3072 (144 / 192) 21.6 /
+// 20.7; 2048 x 3072 -> 9216 and 4096 x 3072 -> 4608 (288 / 384) 48.7 / 42.1 and
+// 47.5 / 41.7; 2304 x 8192 -> 8192 (288 / 387) 108.6 / 90.5; 4096 x 3072 -> 6144
+// (384 / 512) 52.8 / 49.0; with a round more 4608 x 3072 -> 3072 (216 / 288) 28.6 /
+// 43.3, 4608 x 3072 -> 9216 (648 / 864) 82.2 / 93.2, 16384 x 3840 -> 15360 515 /
+// 573.
+int gemm_bf6_large_shape(int M, int N, int K) {
+    (void)K;
+    const long long tm = (M + 255) / 256;
+    const long long r256 = (tm * ((N + 255) / 256) + 255) / 256, r192 = (tm * ((N + 191) / 192) + 255) / 256;
+    return r192 <= r256 ? 192 : 256;
+}
+
 // The workgroup tile (rows of A x rows of B) of a bf6 GEMM launch.
 void gemm_bf6_tile(int M, int N, int K, int nsplit, int* bm, int* bn) {
     *bm = 0;
     if (nsplit <= 1) gemm_bf6_direct_tile(M, N, K, bm, bn);
     if (*bm) return;
-    if (!gemm_bf6_small_tiles(M, N, K)) { *bm = B6_BM; *bn = B6_BN; return; }
+    if (!gemm_bf6_small_tiles(M, N, K)) {
+        *bm = B6_BM;
+        *bn = nsplit <= 1 ? gemm_bf6_large_shape(M, N, K) : B6_BN;
+        return;
+    }
     *bm = 128;
     *bn = gemm_bf6_small_shape(M, N, K, nsplit) == SMALL_128x192 ? 192 : 128;
 }

@@ -192,7 +192,8 @@ int cr_max_quant_bf6_k(void);
 /* cr_int4_convrot_gemm_ex on B6T operands (A6 from M rows, W6 from N rows); epilogue 0..3.
  * At most 256 rows run on tiles of 32 x 32 to 128 x 64 where these fill the CUs
  * once, other grids of at most 512 128 x 128 output tiles with K <= 4096 on 128 x
- * 128 tiles, larger ones on 256 x 256 tiles; the outputs are the same bits. */
+ * 128 tiles, larger ones on 256 x 256 or 256 x 192 tiles; the outputs are the same
+ * bits. */
 int cr_int4_convrot_gemm_bf6(const void* A6, const void* W6, const void* xscale, const void* wscale,
                              const void* bias, void* out, int M, int N, int K, int epilogue, void* stream);
 
@@ -228,7 +229,7 @@ int cr_int4_convrot_gemm_bf6_splitk(const void* A6, const void* W6, const void* 
 int cr_gemm_bf6_choose_nsplit(int M, int N, int K);
 
 /* The workgroup tile (*bm rows of A x *bn rows of B) of a bf6 GEMM launch of
- * M x N x K split nsplit ways: 256 x 256 on large grids, 128 x 128 or 128 x 192
+ * M x N x K split nsplit ways: 256 x 256 or 256 x 192 on large grids, 128 x 128 or 128 x 192
  * on small ones, 32 x 32 to 128 x 64 on unsplit ones of at most 256 rows (the
  * outputs are the same bits whichever runs).  0, or -1 for
  * arguments no launch accepts.  No counterpart in the reference: for tests and
