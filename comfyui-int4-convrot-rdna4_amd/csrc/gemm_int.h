@@ -130,16 +130,20 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
         if (t == 1) read_one(st, s, 3, f);
         if (t == 2) read_one(st, s, 1, f);
     };
-    // slot t (0..3) of a k step: A tile t / 2 against B tile t % 2 (transposed)
+    // slot t of a k step: A tile (t / 2) % 2 against B tile t % 2 (transposed).  Packed
+    // int4 has eight: the first 8 bytes of every fragment, then the last 8, so that
+    // four MFMAs lie between two on one accumulator (1024 x 1600 -> 4800 16.1 -> 15.5
+    // us against the two halves back to back, MI355X).
+    constexpr int SLOTS = KIND == KIND_P4 ? 8 : 4;
     auto lo = [](v4u_d x) { return (v4i){(int)((x.x << 4) & 0xF0F0F0F0u), (int)(x.x & 0xF0F0F0F0u),
                                          (int)((x.y << 4) & 0xF0F0F0F0u), (int)(x.y & 0xF0F0F0F0u)}; };
     auto hi = [](v4u_d x) { return (v4i){(int)((x.z << 4) & 0xF0F0F0F0u), (int)(x.z & 0xF0F0F0F0u),
                                          (int)((x.w << 4) & 0xF0F0F0F0u), (int)(x.w & 0xF0F0F0F0u)}; };
     auto mfma_slot = [&](const Frags& f, int t) __attribute__((always_inline)) {
-        const int i = t >> 1, j = t & 1;
+        const int i = (t >> 1) & 1, j = t & 1;
         if constexpr (KIND == KIND_P4) {
-            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(lo(f.b[j]), lo(f.a[i]), acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(hi(f.b[j]), hi(f.a[i]), acc[i][j], 0, 0, 0);
+            if (t < 4) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(lo(f.b[j]), lo(f.a[i]), acc[i][j], 0, 0, 0);
+            else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(hi(f.b[j]), hi(f.a[i]), acc[i][j], 0, 0, 0);
         } else {
             acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, f.b[j]),
                                                              __builtin_bit_cast(v4i, f.a[i]), acc[i][j], 0, 0, 0);
@@ -163,10 +167,10 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
     for (int kb = 0; kb < nkb; ++kb) {
         const uint32_t st_nxt = st_cur == (NST - 1) * S::STAGE ? 0u : st_cur + S::STAGE;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < SLOTS; ++t) {
             mfma_slot(F0, t);
             __builtin_amdgcn_sched_barrier(0);
-            if (t >= 1) dma_part(kb + NST - 1, t, LOADS_B, LOADS_A);
+            if (t >= 1 && t < 4) dma_part(kb + NST - 1, t, LOADS_B, LOADS_A);
             reads_after(t, st_cur, 1, F1);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -176,10 +180,10 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
         __builtin_amdgcn_sched_barrier(0);
         if (KIND == KIND_P4 && half && kb == nkb - 1) break;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < SLOTS; ++t) {
             mfma_slot(F1, t);
             __builtin_amdgcn_sched_barrier(0);
-            if (t >= 1) dma_part(kb + NST, t, 0, LOADS_B);
+            if (t >= 1 && t < 4) dma_part(kb + NST, t, 0, LOADS_B);
             reads_after(t, st_nxt, 0, F0);
             __builtin_amdgcn_sched_barrier(0);
         }

@@ -3,6 +3,8 @@
 
 #include "gemm_int.h"
 
+#include <algorithm>
+
 namespace convrot {
 
 hipError_t gemm_i8t_large_launch(const int8_t* X, const int8_t* W, const float* xs, const float* ws, const void* bias,
@@ -20,8 +22,9 @@ static long long up(int v, int t) { return (long long)((v + t - 1) / t); }
 // - / 13.4 / 8.4 / 4.6; 256 x 3072 -> 3072 - / 13.7 / 8.0 / 9.5; 512 x 3072 ->
 // 3072 - / 13.8 / 13.2 / 15.5; 512 x 3072 -> 12288 and 2048 x 3072 -> 3072 20.5 on
 // 128 x 128 (384 workgroups); 512 x 12288 -> 3072 100.6 / 43.6, split in two
-// 29.3, in four 27.6 (64 x 64 44.6); 256 x 12288 -> 3072 28.2 split in two, 20.7
-// in four, 23.4 on 64 x 64; 1024 x 12288 -> 3072 44.1, split in two 42.5; 1333 x
+// 29.3, in four 27.6 (64 x 64 44.6); 300 x 12288 -> 3072 (72 tiles)
+// 42.8, in two 28.3, in three 23.4, in four (288 workgroups) 28.7; 256 x 12288 ->
+// 3072 28.2 split in two, 20.7 in four, 23.4 on 64 x 64; 1024 x 12288 -> 3072 44.1, split in two 42.5; 1333 x
 // 2304 -> 6912 (594 workgroups) 25.6 against about 24 on 256 x 256.
 enum : int { I8_LARGE = 0, I8_RING = 1, I8_D64 = 2, I8_D32 = 3 };
 static int i8t_plan(int M, int N, int K, int* nsplit) {
@@ -30,7 +33,7 @@ static int i8t_plan(int M, int N, int K, int* nsplit) {
     if (t32 <= 256 || (t32 <= 512 && K <= 4096)) return I8_D32;
     if (t64 <= 256 && K <= 4096) return I8_D64;
     if (t128 > 512) return I8_LARGE;
-    if (K >= 64 * 96) *nsplit = t128 <= 64 ? 4 : t128 <= 128 ? 2 : 1;
+    if (K >= 64 * 96) *nsplit = (int)std::max(1ll, std::min(4ll, 256 / t128));   // one workgroup per CU
     return I8_RING;
 }
 
