@@ -1,4 +1,4 @@
-// Int8-MFMA GEMM on 64 UA x 64 UB tiles of UA UB waves (64 x 64 outputs each):
+// Int8-MFMA GEMM on 64 UA x 64 UB tiles of waves of 64 x 64 or 128 x 64 outputs:
 // the W8A8 GEMM on grids the 256 x 256 kernel leaves mostly idle, and the
 // packed-int4 GEMM of widths that are no multiple of 128.
 //
@@ -28,11 +28,14 @@ namespace convrot {
 
 constexpr int IN_UNIT = 4096;                            // 64 rows x 64 bytes
 
-template <int UA, int UB, int NST_>
+// FM: 32-row tiles of A per wave (2: 64 x 64 outputs, 4: 128 x 64, which reads a
+// quarter fewer fragment bytes per product; packed int4 keeps 2: with one wave per
+// SIMD nothing hides the unpack, 1024 x 1600 -> 4800 15.3 us against 18.5).
+template <int UA, int UB, int NST_, int FM = 2>
 struct IntTile {
     static constexpr int NST = NST_;
     static constexpr int BM = 64 * UA, BN = 64 * UB;
-    static constexpr int WAVES = UA * UB, THREADS = 64 * WAVES;
+    static constexpr int WAVES = UA * UB * 2 / FM, THREADS = 64 * WAVES;
     static constexpr int STAGE = (UA + UB) * IN_UNIT;
     static constexpr int LOADS = 4 * (UA + UB) / WAVES;  // copies per wave and block
     static constexpr int RING = NST * STAGE;
@@ -42,12 +45,13 @@ struct IntTile {
     static_assert(RING / WAVES >= 32 * (64 * 4 + 16), "epilogue scratch");
 };
 
-template <int KIND, int EPI, int LR, bool SPLIT, int UA, int UB, int NST_>
-__global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
+template <int KIND, int EPI, int LR, bool SPLIT, int UA, int UB, int NST_, int FM>
+__global__ __launch_bounds__(128 * UA * UB / FM) void gemm_int_kernel(
         const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const float* __restrict__ xs,
         const float* __restrict__ ws, const void* __restrict__ bias, int bias_dt, void* __restrict__ out, int M, int N,
         int K, LoraArgs lora, int gm, int nsplit, int* __restrict__ part, unsigned* __restrict__ cnt) {
-    using S = IntTile<UA, UB, NST_>;
+    using S = IntTile<UA, UB, NST_, FM>;
+    static_assert(FM == 2 || !SPLIT, "the partial exchange is laid out for 64 x 64 waves");
     constexpr int NST = S::NST;
     extern __shared__ __attribute__((aligned(16))) uint8_t ilds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -107,42 +111,42 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
         for (int j = n * (t - 1) / 3; j < n * t / 3; ++j) dma_one(kb, first + j);
     };
 
-    v16i acc[2][2];
+    v16i acc[FM][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = (v16i){0};
     const int l32 = lane & 31, h = lane >> 5;
     uint32_t offa[2], offb[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        offa[s] = wm * IN_UNIT + i8t_off(l32, 2 * s + h);
+        offa[s] = wm * (FM / 2) * IN_UNIT + i8t_off(l32, 2 * s + h);
         offb[s] = (UA + wn) * IN_UNIT + i8t_off(l32, 2 * s + h);
     }
-    struct Frags { v4u_d a[2], b[2]; };
+    struct Frags { v4u_d a[FM], b[2]; };
     auto read_one = [&](uint32_t st, int s, int r, Frags& f) __attribute__((always_inline)) {
         const uint8_t* base = ilds + st;
-        if (r < 2) f.a[r] = *reinterpret_cast<const v4u_d*>(base + offa[s] + r * 2048);
-        else f.b[r - 2] = *reinterpret_cast<const v4u_d*>(base + offb[s] + (r - 2) * 2048);
+        if (r < FM) f.a[r] = *reinterpret_cast<const v4u_d*>(base + offa[s] + r * 2048);
+        else f.b[r - FM] = *reinterpret_cast<const v4u_d*>(base + offb[s] + (r - FM) * 2048);
     };
     auto reads_after = [&](int t, uint32_t st, int s, Frags& f) __attribute__((always_inline)) {
-        if (t == 0) { read_one(st, s, 0, f); read_one(st, s, 2, f); }
-        if (t == 1) read_one(st, s, 3, f);
-        if (t == 2) read_one(st, s, 1, f);
+        if (t == 0) { read_one(st, s, 0, f); read_one(st, s, FM, f); }
+        if (t == 1) read_one(st, s, FM + 1, f);
+        if (t >= 2 && t <= FM) read_one(st, s, t - 1, f);
     };
-    // slot t of a k step: A tile (t / 2) % 2 against B tile t % 2 (transposed).  Packed
-    // int4 has eight: the first 8 bytes of every fragment, then the last 8, so that
+    // slot t of a k step: A tile (t / 2) % FM against B tile t % 2 (transposed).  Packed
+    // int4 has twice as many: the first 8 bytes of every fragment, then the last 8, so that
     // four MFMAs lie between two on one accumulator (1024 x 1600 -> 4800 16.1 -> 15.5
     // us against the two halves back to back, MI355X).
-    constexpr int SLOTS = KIND == KIND_P4 ? 8 : 4;
+    constexpr int SLOTS = KIND == KIND_P4 ? 4 * FM : 2 * FM;
     auto lo = [](v4u_d x) { return (v4i){(int)((x.x << 4) & 0xF0F0F0F0u), (int)(x.x & 0xF0F0F0F0u),
                                          (int)((x.y << 4) & 0xF0F0F0F0u), (int)(x.y & 0xF0F0F0F0u)}; };
     auto hi = [](v4u_d x) { return (v4i){(int)((x.z << 4) & 0xF0F0F0F0u), (int)(x.z & 0xF0F0F0F0u),
                                          (int)((x.w << 4) & 0xF0F0F0F0u), (int)(x.w & 0xF0F0F0F0u)}; };
     auto mfma_slot = [&](const Frags& f, int t) __attribute__((always_inline)) {
-        const int i = (t >> 1) & 1, j = t & 1;
+        const int i = (t >> 1) % FM, j = t & 1;
         if constexpr (KIND == KIND_P4) {
-            if (t < 4) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(lo(f.b[j]), lo(f.a[i]), acc[i][j], 0, 0, 0);
+            if (t < 2 * FM) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(lo(f.b[j]), lo(f.a[i]), acc[i][j], 0, 0, 0);
             else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(hi(f.b[j]), hi(f.a[i]), acc[i][j], 0, 0, 0);
         } else {
             acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, f.b[j]),
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
 #pragma unroll
     for (int j = 0; j < LOADS_B; ++j) dma_one(NST - 1, j);         // the rest in phase A of block 0
 #pragma unroll
-    for (int r = 0; r < 4; ++r) read_one(0, 0, r, F0);
+    for (int r = 0; r < FM + 2; ++r) read_one(0, 0, r, F0);
     // packed int4: the last block holds one k step only when K % 128 == 64
     const bool half = KIND == KIND_P4 && Kb % 64 != 0;
     uint32_t st_cur = 0;
@@ -224,17 +228,17 @@ __global__ __launch_bounds__(64 * UA * UB) void gemm_int_kernel(
     scr.store(sc, bias, bias_dt, M, N, m0, n0, tid);
     __syncthreads();
     constexpr int SCR = S::RING / S::WAVES;
-    epilogue_lds<EPI, 2, 2, LR, SCR, KIND == KIND_P4 ? 8 : 0, true>(acc, sc, out, M, N, m0, n0, m0 + wm * 64,
+    epilogue_lds<EPI, FM, 2, LR, SCR, KIND == KIND_P4 ? 8 : 0, true>(acc, sc, out, M, N, m0, n0, m0 + wm * 32 * FM,
                                                                     n0 + wn * 64, lane, lora, ilds + wave * SCR);
 }
 
 // One launch, split nsplit ways (nsplit > 1: part holds nsplit partials per tile, cnt one counter).
-template <int KIND, int EPI, int LR, bool SPLIT, int UA, int UB, int NST>
+template <int KIND, int EPI, int LR, bool SPLIT, int UA, int UB, int NST, int FM = 2>
 static hipError_t int_launch(const uint8_t* A, const uint8_t* B, const float* xs, const float* ws, const void* bias,
                              int bias_dt, void* out, int M, int N, int K, const LoraArgs& la, int nsplit, int* part,
                              unsigned* cnt, int dev, hipStream_t st) {
-    using S = IntTile<UA, UB, NST>;
-    auto kern = &gemm_int_kernel<KIND, EPI, LR, SPLIT, UA, UB, NST>;
+    using S = IntTile<UA, UB, NST, FM>;
+    auto kern = &gemm_int_kernel<KIND, EPI, LR, SPLIT, UA, UB, NST, FM>;
     static std::atomic<bool> attr[kMaxDev];
     const hipError_t e = lds_limit_once(attr, dev, reinterpret_cast<const void*>(kern), S::LDS_BYTES);
     if (e != hipSuccess) return e;

@@ -12,8 +12,8 @@ hipError_t gemm_i8t_large_launch(const int8_t* X, const int8_t* W, const float* 
 
 static long long up(int v, int t) { return (long long)((v + t - 1) / t); }
 
-// Kernel of a W8A8 product: the 256 x 256 tiles (gemm.hip), the 128 x 128 ring
-// split nsplit ways, or the direct kernel on 64 x 64 or 32 x 32 tiles.  A
+// Kernel of a W8A8 product: the 256 x 256 tiles (gemm.hip), the 256 x 128 ring,
+// the 128 x 128 ring split nsplit ways, or the direct kernel on 64 x 64 or 32 x 32 tiles.  A
 // workgroup's time is its operand bytes at the rate of one CU, so the tile
 // shrinks until the grid covers the CUs; the direct tiles read more bytes per
 // product and win only while k is short or the grid tiny; a split's exchange
@@ -25,14 +25,20 @@ static long long up(int v, int t) { return (long long)((v + t - 1) / t); }
 // 29.3, in four 27.6 (64 x 64 44.6); 300 x 12288 -> 3072 (72 tiles)
 // 42.8, in two 28.3, in three 23.4, in four (288 workgroups) 28.7; 256 x 12288 ->
 // 3072 28.2 split in two, 20.7 in four, 23.4 on 64 x 64; 1024 x 12288 -> 3072 44.1, split in two 42.5; 1333 x
-// 2304 -> 6912 (594 workgroups) 25.6 against about 24 on 256 x 256.
-enum : int { I8_LARGE = 0, I8_RING = 1, I8_D64 = 2, I8_D32 = 3 };
+// 2304 -> 6912 (594 workgroups) 25.6 against about 24 on 256 x 256.  Between
+// one and two 128 x 128 workgroups per CU, 256 x 128 tiles of four 128 x 64 waves
+// where these fit one per CU (uniform codes, 256 x 256 / 128 x 128 / 256 x 128 of
+// 64 x 64 waves / of 128 x 64 waves): 2048 x 3072 -> 3072 33.5 / 26.4 / 25.0 / 23.7,
+// 2048 x 12288 -> 3072 102.5 / 90.5 / 84.2 / 77.6; above that the 256 x 256 kernel:
+// 4096 x 3072 -> 3072 40.8 / 45.0 / 50.3 / 47.9.
+enum : int { I8_LARGE = 0, I8_RING = 1, I8_D64 = 2, I8_D32 = 3, I8_WIDE = 4 };
 static int i8t_plan(int M, int N, int K, int* nsplit) {
     const long long t32 = up(M, 32) * up(N, 32), t64 = up(M, 64) * up(N, 64), t128 = up(M, 128) * up(N, 128);
     *nsplit = 1;
     if (t32 <= 256 || (t32 <= 512 && K <= 4096)) return I8_D32;
     if (t64 <= 256 && K <= 4096) return I8_D64;
     if (t128 > 512) return I8_LARGE;
+    if (t128 > 256 && up(M, 256) * up(N, 128) <= 256) return I8_WIDE;
     if (K >= 64 * 96) *nsplit = (int)std::max(1ll, std::min(4ll, 256 / t128));   // one workgroup per CU
     return I8_RING;
 }
@@ -56,6 +62,7 @@ static hipError_t i8t_run(const uint8_t* A, const uint8_t* B, const float* xs, c
     switch (i8t_plan(M, N, K, &ns)) {
         case I8_D32: return direct_launch<KIND_I8T, EPI, false, 1, 1, 1, 1, 8, 4>(A, B, xs, ws, bias, bias_dt, out, M, N, K, none, dev, st);
         case I8_D64: return direct_launch<KIND_I8T, EPI, false, 2, 2, 1, 1, 8, 2>(A, B, xs, ws, bias, bias_dt, out, M, N, K, none, dev, st);
+        case I8_WIDE: return int_launch<KIND_I8T, EPI, 0, false, 4, 2, 4, 4>(A, B, xs, ws, bias, bias_dt, out, M, N, K, none, 1, nullptr, nullptr, dev, st);
         case I8_RING: break;
         default: return gemm_i8t_large_launch(reinterpret_cast<const int8_t*>(A), reinterpret_cast<const int8_t*>(B), xs, ws, bias, bias_dt, out, M, N, K, EPI, st);
     }
