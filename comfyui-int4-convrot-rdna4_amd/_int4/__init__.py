@@ -233,10 +233,13 @@ def convrot_w4a4_linear(
     GEMM's.  Without it, inputs whose K allows it still take the bf6 GEMM with
     the weight re-encoded on the fly.
 
-    Two kernels per call, both on torch's current stream: the fused
-    rotate+quantize of x, then the W4A4 GEMM with the dequant epilogue.  Every
-    row count takes the same kernels (the reference's torch-rotation branch
-    for M < 512 is not needed: the fused kernel is exact and fast at any M).
+    Two stages per call, both on torch's current stream: the fused
+    rotate+quantize of x, then the W4A4 GEMM with the dequant epilogue, on the
+    tile its grid fills the GPU with.  Every row count takes them (the
+    reference's torch-rotation branch for M < 512 is not needed: the fused
+    kernel is exact and fast at any M).  Contiguous GPU operands go through
+    the native host path (csrc/host.cpp), every other form through the steps
+    below, with the same results.
 
     linear_dtype "int8" marks layers the reference sends to its eager path
     (_int4/__init__.py:104-111 -> _int4/eager.py:172-197), whose output is the

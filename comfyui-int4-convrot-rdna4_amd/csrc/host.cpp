@@ -10,7 +10,7 @@
 // workgroups need a workspace with cleared counters and are left to Python,
 // which keeps one per stream.
 //
-// Measured on an MI355X box (M = 1, 256 x 256, back to back): 17.3 us per W4A4
+// Measured on MI355X (M = 1, 256 x 256, back to back): 17.3 us per W4A4
 // call through Python and ctypes, 7.1 here; 21.9 and 9.5 with a LoRA; W8A8 27.2
 // (16.0 as one library call) and 6.8.
 
