@@ -194,6 +194,17 @@ _MAX_WORKSPACES = 16
 SPLIT_COUNTER_BYTES = 2048
 _workspaces: "collections.OrderedDict" = collections.OrderedDict()
 _workspaces_lock = threading.Lock()
+# A call queues several launches that hand the codes, the row scales and the
+# partials on in the workspace, and the library call runs without the GIL: from
+# the lookup to the last launch a thread holds its stream's lock, so that the
+# calls of threads that share a stream (the default one is every thread's) are
+# queued one whole call after the other.  A fixed set: a lock is never dropped
+# while a thread holds it, and streams that share one only queue in turn.
+_call_locks = tuple(threading.RLock() for _ in range(64))
+
+
+def _call_lock(device, stream: int):
+    return _call_locks[hash((device.index, stream)) % len(_call_locks)]
 
 
 def _new_workspace(device, nbytes: int) -> torch.Tensor:
@@ -385,8 +396,9 @@ def lora_down(x: torch.Tensor, down: torch.Tensor) -> torch.Tensor:
         return t
     nbytes = lib.cr_lora_down_workspace(M, K, R)        # 0 for an unsplit shape
     st = _stream(x.device)
-    ws = _workspace(x.device, st, nbytes)
-    rc = lib.cr_lora_down(_ptr(x), _IN_DTYPE_CODE[x.dtype], _ptr(down), _ptr(t), M, K, R, _ptr(ws), nbytes, st)
+    with _call_lock(x.device, st):
+        ws = _workspace(x.device, st, nbytes)
+        rc = lib.cr_lora_down(_ptr(x), _IN_DTYPE_CODE[x.dtype], _ptr(down), _ptr(t), M, K, R, _ptr(ws), nbytes, st)
     if rc != 0:
         raise RuntimeError(f"cr_lora_down failed, hipError={rc}")
     return t
@@ -532,10 +544,11 @@ def _bf6_launch(a6, w6, xs, wsc, b, t, up, R, scale, out, M, N, K, epilogue, nsp
             name = "cr_int4_convrot_gemm_bf6_lora"
     else:
         nbytes = lib.cr_gemm_bf6_splitk_workspace(M, N, nsplit)
-        ws = _workspace(a6.device, st, nbytes)
-        rc = lib.cr_int4_convrot_gemm_bf6_splitk(_ptr(a6), _ptr(w6), _ptr(xs), _ptr(wsc), _ptr(b), _ptr(t),
-                                                 _ptr(up), R, ctypes.c_float(scale), _ptr(out), M, N, K, epilogue,
-                                                 nsplit, _ptr(ws), nbytes, st)
+        with _call_lock(a6.device, st):
+            ws = _workspace(a6.device, st, nbytes)
+            rc = lib.cr_int4_convrot_gemm_bf6_splitk(_ptr(a6), _ptr(w6), _ptr(xs), _ptr(wsc), _ptr(b), _ptr(t),
+                                                     _ptr(up), R, ctypes.c_float(scale), _ptr(out), M, N, K, epilogue,
+                                                     nsplit, _ptr(ws), nbytes, st)
         name = "cr_int4_convrot_gemm_bf6_splitk"
     if rc != 0:
         raise RuntimeError(f"{name} failed, hipError={rc}")
@@ -769,13 +782,14 @@ def convrot_w4a4_linear_bf6(x2d, w6, w_scale, bias, down, up, scale: float, epil
     R = 0 if down is None else down.shape[0]
     nbytes = lib.cr_convrot_w4a4_linear_bf6_workspace(M, N, K, R)
     st = _stream(x2d.device)
-    ws = _workspace(x2d.device, st, nbytes)
     bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
     head = (_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w6), _ptr(w_scale), _ptr(bias), bdt, _ptr(down), _ptr(up), R,
             scale, _ptr(out))
-    tail = (M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
-    rc = lib.cr_convrot_w4a4_linear_bf6_f16(*head, *tail) if epilogue == EPI_F16 else \
-        lib.cr_convrot_w4a4_linear_bf6(*head, epilogue, *tail)
+    with _call_lock(x2d.device, st):
+        ws = _workspace(x2d.device, st, nbytes)
+        tail = (M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+        rc = lib.cr_convrot_w4a4_linear_bf6_f16(*head, *tail) if epilogue == EPI_F16 else \
+            lib.cr_convrot_w4a4_linear_bf6(*head, epilogue, *tail)
     if rc != 0:
         raise RuntimeError(f"cr_convrot_w4a4_linear_bf6 failed, hipError={rc}")
     return out
@@ -792,11 +806,12 @@ def convrot_w4a4_linear_packed(x2d, qweight, w_scale, bias, down, up, scale: flo
     R = 0 if down is None else down.shape[0]
     nbytes = lib.cr_convrot_w4a4_linear_packed_workspace(M, N, K, R)
     st = _stream(x2d.device)
-    ws = _workspace(x2d.device, st, nbytes)
     bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
-    rc = lib.cr_convrot_w4a4_linear_packed(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(qweight), _ptr(w_scale),
-                                           _ptr(bias), bdt, _ptr(down), _ptr(up), R, scale, _ptr(out), epilogue,
-                                           M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    with _call_lock(x2d.device, st):
+        ws = _workspace(x2d.device, st, nbytes)
+        rc = lib.cr_convrot_w4a4_linear_packed(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(qweight), _ptr(w_scale),
+                                               _ptr(bias), bdt, _ptr(down), _ptr(up), R, scale, _ptr(out), epilogue,
+                                               M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
     if rc != 0:
         raise RuntimeError(f"cr_convrot_w4a4_linear_packed failed, hipError={rc}")
     return out
@@ -814,10 +829,11 @@ def convrot_w8a8_linear_i8t(x2d, w8t, w_scale, bias, epilogue: int, convrot_grou
     out = torch.empty((M, N), dtype=_OUT_DTYPE[epilogue], device=x2d.device)
     nbytes = lib.cr_convrot_w8a8_linear_i8t_workspace(M, N, K)
     st = _stream(x2d.device)
-    ws = _workspace(x2d.device, st, nbytes)
     bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
-    rc = lib.cr_convrot_w8a8_linear_i8t(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w8t), _ptr(w_scale), _ptr(bias),
-                                        bdt, _ptr(out), epilogue, M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
+    with _call_lock(x2d.device, st):
+        ws = _workspace(x2d.device, st, nbytes)
+        rc = lib.cr_convrot_w8a8_linear_i8t(_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w8t), _ptr(w_scale), _ptr(bias),
+                                            bdt, _ptr(out), epilogue, M, N, K, convrot_groupsize, _ptr(ws), nbytes, st)
     if rc != 0:
         raise RuntimeError(f"cr_convrot_w8a8_linear_i8t failed, hipError={rc}")
     return out
