@@ -57,6 +57,25 @@ def test_kernel_infinite_scale(backend, gpu):
     assert bool(y[1].isnan().all()) and bool(y[0].isfinite().all()) and bool(y[2].isfinite().all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [16, 64, 256])
+def test_kernel_infinite_scale_of_one_sign(backend, gpu, G):
+    """An infinite scale times codes that follow a row of H leaves that sum
+    infinite, a zero among the codes or any other order of signs NaN, as the
+    torch composition sums them; a NaN scale leaves NaN."""
+    h = backend._hadamard(G, "cpu")
+    q = (h[3].sign() * 5).to(torch.int8).repeat(5, 2)
+    q[1, 0] = 0
+    q[2, :G] = -q[2, :G]
+    s = torch.tensor([float("inf"), float("inf"), float("-inf"), float("nan"), 0.25])
+    want = torch.matmul((q.float() * s[:, None]).reshape(5, 2, G), h.T).reshape(5, 2 * G)
+    assert int(want.isinf().sum()) == 5                     # 2 + 1 + 2: the third row of H in each group
+    y = dequantize(backend, q.cuda(), s.cuda(), 8, G).cpu()
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(0.0), want.nan_to_num(0.0))
+    z = dequantize(backend, backend._pack_int4_row_major(q).cuda(), s.cuda(), 4, G).cpu()
+    assert torch.equal(z.isnan(), want.isnan()) and torch.equal(z.nan_to_num(0.0), want.nan_to_num(0.0))
+
+
 def test_route_rule(backend, native):
     """CPU tensors and calls under a transform, trace or gradient keep the torch composition."""
     q, s = codes(4, 256, 8, 1)
