@@ -420,6 +420,11 @@ def convrot_w8a8_linear(
         x2d = x2d.to(torch.float32)
     out_dtype = x.dtype if x.dtype in _NATIVE_OUT else torch.float32
     N = qweight.shape[0]
+    # the kernels read N of each
+    if wscales.numel() != N:
+        raise ValueError(f"wscales has {wscales.numel()} elements, the weight has N={N} rows")
+    if bias is not None and bias.numel() != N:
+        raise ValueError(f"bias has {bias.numel()} elements, the weight has N={N} rows")
     if i8t_path_ok(x2d.shape[1]) and x2d.is_cuda:
         w8t = qweight_i8t if qweight_i8t is not None else prepare_convrot_w8a8_weight_i8t(qweight)
         # the bias is read as stored (f32 / bf16 / f16): no conversion launch per call

@@ -193,6 +193,17 @@ def test_linear_validation_errors(backend):
         backend.convrot_w4a4_linear(x, qw, ws, lora=(D, torch.zeros(8, 64, dtype=torch.bfloat16)))
 
 
+@pytest.mark.parametrize("K", [512, 80])                             # the tile-major and the row-major widths
+def test_w8a8_operand_lengths(backend, K):
+    """Scales and bias that are not N long raise before any device work."""
+    x, qw, ws = torch.zeros(4, K, dtype=torch.bfloat16), torch.zeros(8, K, dtype=torch.int8), torch.ones(8)
+    for n in (1, 7, 9):
+        with pytest.raises(ValueError, match="wscales"):
+            backend.convrot_w8a8_linear(x, qw, torch.ones(n), convrot_groupsize=16)
+        with pytest.raises(ValueError, match="bias"):
+            backend.convrot_w8a8_linear(x, qw, ws, bias=torch.zeros(n), convrot_groupsize=16)
+
+
 def test_weight_validation_errors(backend):
     with pytest.raises(ValueError):
         backend.quantize_convrot_w4a4_weight(torch.zeros(8, 512), quant_group_size=32)

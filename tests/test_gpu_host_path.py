@@ -105,6 +105,23 @@ def test_other_forms_go_to_python(backend, native, gpu):
         backend.convrot_w4a4_linear(x, qw, s, bias=b.cpu(), qweight_bf6=w6)
 
 
+def test_w8a8_bad_operands_are_refused(backend, native, gpu):
+    """Lengths and shapes the host module leaves to Python raise there, before any launch."""
+    M, N, K = 48, 384, 256
+    x = outlier_activations(M, K, seed=3).cuda()
+    q = torch.randint(-127, 128, (N, K), generator=torch.Generator().manual_seed(1)).to(torch.int8).cuda()
+    s, b, t = torch.ones(N, device="cuda"), normal_bias(N, seed=5).cuda(), native.int8_to_i8t(q)
+    good = dict(x=x, qweight=q, wscales=s, bias=b, qweight_i8t=t)
+    want = backend.convrot_w8a8_linear(**good)
+    for bad in [dict(wscales=s[:-1]), dict(wscales=s[:1]), dict(bias=b[:-1]), dict(qweight_i8t=t[:-256]),
+                dict(qweight=q[:, :-64]), dict(convrot_groupsize=128)]:
+        with pytest.raises(ValueError):
+            backend.convrot_w8a8_linear(**{**good, **bad})
+    with pytest.raises(RuntimeError):
+        backend.convrot_w8a8_linear(**{**good, "bias": b.cpu()})
+    assert torch.equal(backend.convrot_w8a8_linear(**{**good, "wscales": s[:, None], "bias": b[None]}), want)
+
+
 def test_streams_and_threads(backend, native, gpu):
     """Calls on several streams from several threads: their intermediates never meet."""
     import threading
