@@ -42,11 +42,13 @@ def _deps() -> list[str]:
 
 
 def is_stale() -> bool:
-    out = lib_path()
-    if not os.path.exists(out) or not os.path.exists(host_path()):
+    """Whether a source is newer than what was built from it, or the host module
+    older than the library it is linked to (a build that ended between the two)."""
+    out, host = lib_path(), host_path()
+    if not os.path.exists(out) or not os.path.exists(host):
         return True
     t = os.path.getmtime(out)
-    return any(os.path.getmtime(d) > t for d in _deps() if os.path.exists(d))
+    return os.path.getmtime(host) < t or any(os.path.getmtime(d) > t for d in _deps() if os.path.exists(d))
 
 
 def _hipcc() -> str:
@@ -105,16 +107,14 @@ def _compile_host() -> str:
     return obj
 
 
-def _link_host(obj: str, lib: str) -> None:
+def _link_host(obj: str, lib: str, out: str) -> None:
     """The CPython module, bound to the kernel library next to it."""
     _run([_hipcc(), "-shared", "-fPIC", "-Wl,--as-needed", obj, "-L" + os.path.join(_torch_dir(), "lib"), "-ltorch_python", "-ltorch_cpu",
           "-lc10", "-lc10_hip", "-L" + os.path.dirname(lib), "-l:" + os.path.basename(lib), "-Wl,-rpath,$ORIGIN"],
-         host_path(), "linking the host module")
+         out, "linking the host module")
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> str:
-    out = lib_path()
-    tmp = out + ".tmp"
     srcs = sources()
     if verbose:
         print("building:", " ".join([_hipcc(), *CFLAGS, "-c", "<src>"]), "for", ", ".join(SOURCES))
@@ -122,13 +122,14 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     with ThreadPoolExecutor(max_workers=n) as ex:
         host = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
-    cp = subprocess.run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp],
-                        capture_output=True, text=True)
-    if cp.returncode != 0 or not os.path.exists(tmp):
-        raise RuntimeError(f"hipcc link failed:\n{cp.stderr}")
-    os.replace(tmp, out)
-    _link_host(host.result(), out)
-    return out
+    # both linked aside under their names, then moved in place: a build that fails leaves the pair that was there
+    lib = os.path.join(_obj_dir(), os.path.basename(lib_path()))
+    mod = os.path.join(_obj_dir(), os.path.basename(host_path()))
+    _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs], lib, "hipcc link")
+    _link_host(host.result(), lib, mod)
+    os.replace(lib, lib_path())
+    os.replace(mod, host_path())
+    return lib_path()
 
 
 if __name__ == "__main__":

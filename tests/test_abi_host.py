@@ -348,6 +348,61 @@ def test_tile_choice(native):
     assert lib.cr_gemm_bf6_tile(1, 1, 128, 1, None, None) == -1
 
 
+@pytest.fixture
+def build_in(native, monkeypatch, tmp_path):
+    """The build module on an empty folder, its compilers replaced by file writers;
+    `fail` names the step that raises."""
+    b, state = native._build, {"fail": None, "n": 0}
+
+    def step(out, what):
+        if state["fail"] and state["fail"] in what:
+            raise RuntimeError(what)
+        state["n"] += 1
+        with open(out, "w") as f:
+            f.write(str(state["n"]))
+        return out
+    monkeypatch.setattr(b, "lib_path", lambda: str(tmp_path / "libk.so"))
+    monkeypatch.setattr(b, "host_path", lambda: str(tmp_path / "h.so"))
+    monkeypatch.setattr(b, "_obj_dir", lambda: (tmp_path / "obj").mkdir(exist_ok=True) or str(tmp_path / "obj"))
+    monkeypatch.setattr(b, "_compile", lambda src: src)
+    monkeypatch.setattr(b, "_compile_host", lambda: step(str(tmp_path / "host.o"), "compile host"))
+
+    def run(cmd, *a, **k):
+        import subprocess
+        step(cmd[cmd.index("-o") + 1], "link " + cmd[cmd.index("-o") + 1])
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+    monkeypatch.setattr(b.subprocess, "run", run)
+    return b, state, tmp_path
+
+
+@pytest.mark.parametrize("fail", ["compile host", "h.so", "libk.so"])
+def test_failed_build_leaves_the_pair(build_in, fail):
+    """The kernel library and the host module bound to it are replaced together or not at all."""
+    b, state, tmp = build_in
+    b.build(jobs=2)
+    before = [(tmp / n).read_text() for n in ("libk.so", "h.so")]
+    state["fail"] = fail
+    with pytest.raises(RuntimeError):
+        b.build(jobs=2)
+    assert [(tmp / n).read_text() for n in ("libk.so", "h.so")] == before
+
+
+def test_stale_host_module(build_in):
+    """A host module older than the library, or none, is stale however new the library is."""
+    import os
+    import time
+    b, _, tmp = build_in
+    b.build(jobs=2)
+    now = time.time() + 100
+    os.utime(tmp / "libk.so", (now, now))
+    os.utime(tmp / "h.so", (now, now))
+    assert not b.is_stale()
+    os.utime(tmp / "h.so", (now - 10, now - 10))
+    assert b.is_stale()
+    (tmp / "h.so").unlink()
+    assert b.is_stale()
+
+
 def test_ops_meta_skeleton(ops_mod):
     """skeleton_meta_init builds meta-device parameters (the loader's LoRA
     key-map discovery pass) with the quantized-state attributes unset."""
