@@ -133,6 +133,10 @@ def host_module():
                 spec = importlib.util.spec_from_file_location("_host", path, loader=loader)
                 mod = importlib.util.module_from_spec(spec)
                 loader.exec_module(mod)
+                if getattr(mod, "ABI_VERSION", None) != ABI_VERSION:
+                    raise RuntimeError(f"{os.path.basename(path)} was built for ABI version "
+                                       f"{getattr(mod, 'ABI_VERSION', None)}, these bindings need {ABI_VERSION}; "
+                                       "rebuild it with the package's _int4/build.py")
                 _host = mod
     return _host
 

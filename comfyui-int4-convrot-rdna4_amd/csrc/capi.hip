@@ -511,4 +511,4 @@ API int cr_convrot_dequant(const void* q, int bits, const void* scale, void* out
 
 API int cr_max_quant_k(void) { return convrot::rotquant_max_k(); }
 
-API int cr_abi_version(void) { return 13; }
+API int cr_abi_version(void) { return CR_ABI_VERSION; }

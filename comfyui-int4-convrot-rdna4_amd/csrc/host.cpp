@@ -212,4 +212,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+// ABI_VERSION: of the library's signatures this module was compiled with.
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", CR_ABI_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

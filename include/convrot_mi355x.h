@@ -35,6 +35,10 @@
 
 #include <stddef.h>
 
+/* The ABI version of this header (increments on any signature change); cr_abi_version()
+ * returns the library's. */
+#define CR_ABI_VERSION 13
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -392,7 +396,7 @@ int cr_max_quant_k(void);
 int cr_convrot_dequant(const void* q, int bits, const void* scale, void* out, int out_dtype, int N, int K, int G,
                        void* stream);
 
-/* ABI version of this library (increments on any signature change). */
+/* CR_ABI_VERSION of the header this library was built with. */
 int cr_abi_version(void);
 
 #ifdef __cplusplus

@@ -90,6 +90,18 @@ def test_load_refuses_other_abi_version(native, monkeypatch):
         native.load_library()
 
 
+def test_host_module_carries_the_abi_version(native, monkeypatch):
+    """The host module calls the library with compiled-in signatures: bindings for
+    another version, or a module that names none, are refused."""
+    assert native.host_module().ABI_VERSION == native.load_library().cr_abi_version()
+    native.load_library()
+    monkeypatch.setattr(native, "_host", None)
+    monkeypatch.setattr(native, "ABI_VERSION", native.ABI_VERSION + 1)
+    with pytest.raises(RuntimeError, match="ABI version"):
+        native.host_module()
+    assert native._host is None
+
+
 def test_library_queries_without_gpu(native):
     lib = native.load_library()
     assert lib.cr_abi_version() == native.ABI_VERSION == 13
