@@ -252,8 +252,9 @@ def convrot_w4a4_linear(
     """
     if type(x) is torch.Tensor and x.is_cuda and quant_group_size == _INT4_GROUP_SIZE \
             and linear_dtype in ("int4", "int8"):
-        y = native.host_module().w4a4(x, qweight, wscales, bias, convrot_groupsize, linear_dtype == "int8", lora,
-                                      qweight_bf6)
+        host = native.host_or_none()
+        y = None if host is None else host.w4a4(x, qweight, wscales, bias, convrot_groupsize, linear_dtype == "int8",
+                                                lora, qweight_bf6)
         if y is not None:
             return y
     # every form the native host path leaves
@@ -405,7 +406,8 @@ def convrot_w8a8_linear(
     once at load time; re-laid here when not given): the same codes and
     accumulators, bit-identical outputs."""
     if type(x) is torch.Tensor and x.is_cuda:
-        y = native.host_module().w8a8(x, qweight, wscales, bias, convrot_groupsize, qweight_i8t)
+        host = native.host_or_none()
+        y = None if host is None else host.w8a8(x, qweight, wscales, bias, convrot_groupsize, qweight_i8t)
         if y is not None:
             return y
     if x.shape[-1] != qweight.shape[-1]:

@@ -15,6 +15,7 @@ import collections
 import ctypes
 import importlib.machinery
 import importlib.util
+import logging
 import os
 import threading
 
@@ -139,6 +140,27 @@ def host_module():
                                        "rebuild it with the package's _int4/build.py")
                 _host = mod
     return _host
+
+
+_host_error = None
+
+
+def host_or_none():
+    """The host module for the linears, or None where it is missing or does not
+    load (it is bound to torch's C++ ABI, the kernel library is not): said once,
+    and the Python path makes the same launches at 10 us more per call."""
+    global _host_error
+    if _host is not None:
+        return _host
+    load_library()                           # without the kernels there is no other path
+    if _host_error is None:
+        try:
+            return host_module()
+        except Exception as e:
+            _host_error = e
+            logging.warning("ConvRot: %s does not load, the linears run through Python: %s",
+                            os.path.basename(_build.host_path()), e)
+    return None
 
 
 def exported_symbols() -> list[str]:

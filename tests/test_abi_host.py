@@ -102,6 +102,25 @@ def test_host_module_carries_the_abi_version(native, monkeypatch):
     assert native._host is None
 
 
+@pytest.mark.parametrize("kind", ["missing", "broken"])
+def test_linears_run_without_the_host_module(native, monkeypatch, tmp_path, caplog, kind):
+    """No host module, or one that does not import: said once, and the linears
+    take their Python path; without the kernel library they raise."""
+    path = tmp_path / "_host.so"
+    if kind == "broken":
+        path.write_bytes(b"not a library")
+    monkeypatch.setattr(native._build, "host_path", lambda: str(path))
+    monkeypatch.setattr(native, "_host", None)
+    monkeypatch.setattr(native, "_host_error", None)
+    with caplog.at_level("WARNING"):
+        assert native.host_or_none() is None and native.host_or_none() is None
+    assert len(caplog.records) == 1 and "_host.so" in caplog.text
+    monkeypatch.setattr(native, "_lib", None)
+    monkeypatch.setattr(native, "lib_path", lambda: str(tmp_path / "none.so"))
+    with pytest.raises(RuntimeError, match="not built"):
+        native.host_or_none()
+
+
 def test_library_queries_without_gpu(native):
     lib = native.load_library()
     assert lib.cr_abi_version() == native.ABI_VERSION == 13

@@ -62,6 +62,22 @@ def test_w8a8_same_bits(backend, native, gpu, M, N, K, dt):
         assert y.dtype == dt and torch.equal(y, native.convrot_w8a8_linear_i8t(x, t, s, b, epi, 64, N))
 
 
+def test_without_the_host_module(backend, native, gpu, monkeypatch, tmp_path):
+    """The linears answer, bit for bit, where the host module is missing."""
+    x, qw, s, b, G, lora, w6 = setup(backend, 130, 700, 256, torch.bfloat16, 32)
+    q = torch.randint(-127, 128, (700, 256), generator=torch.Generator().manual_seed(2)).to(torch.int8).cuda()
+    t = native.int8_to_i8t(q)
+
+    def both():
+        return (backend.convrot_w4a4_linear(x, qw, s, bias=b, convrot_groupsize=G, lora=lora, qweight_bf6=w6),
+                backend.convrot_w8a8_linear(x, q, s, bias=b, qweight_i8t=t))
+    want = both()
+    monkeypatch.setattr(native._build, "host_path", lambda: str(tmp_path / "_host.so"))
+    monkeypatch.setattr(native, "_host", None)
+    monkeypatch.setattr(native, "_host_error", None)
+    assert all(torch.equal(y, w) for y, w in zip(both(), want))
+
+
 def test_other_forms_go_to_python(backend, native, gpu):
     M, N, K = 48, 384, 256
     x, qw, s, b, G, lora, w6 = setup(backend, M, N, K, torch.bfloat16, 32)
