@@ -68,6 +68,7 @@ _SIGNATURES = {
     "cr_convrot_w4a4_linear_bf6": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                    + [_vp, ctypes.c_size_t, _vp], _i),
     "cr_convrot_w4a4_linear_bf6_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
+    "cr_convrot_w4a4_linear_bf6_min_workspace": ([_i, _i, _i, _i], ctypes.c_size_t),
     "cr_convrot_w4a4_linear_bf6_noalloc": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 5
                                            + [_vp], _i),
     "cr_convrot_w4a4_linear_bf6_f16": ([_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, ctypes.c_float, _vp] + [_i] * 4
@@ -806,7 +807,7 @@ def convrot_w4a4_linear_bf6(x2d, w6, w_scale, bias, down, up, scale: float, epil
     M, K = x2d.shape
     out = torch.empty((M, N), dtype=_OUT_DTYPE[epilogue], device=x2d.device)
     R = 0 if down is None else down.shape[0]
-    nbytes = lib.cr_convrot_w4a4_linear_bf6_workspace(M, N, K, R)
+    nbytes = lib.cr_convrot_w4a4_linear_bf6_min_workspace(M, N, K, R)
     st = _stream(x2d.device)
     bdt = 0 if bias is None else _IN_DTYPE_CODE[bias.dtype]
     head = (_ptr(x2d), _IN_DTYPE_CODE[x2d.dtype], _ptr(w6), _ptr(w_scale), _ptr(bias), bdt, _ptr(down), _ptr(up), R,

@@ -279,27 +279,39 @@ namespace {
 // 0 .. 2047 of every workspace, whatever the shape and split, so that no
 // other intermediate of any call ever overwrites them), then the B6T codes,
 // the row scales, t and the LoRA partials.
-struct LinPlan { size_t part, a6, xs, t, lpart, total; int nsplit; };
+// total: the bytes a call's kernels use; documented: the size the _workspace query
+// states, which also holds the partials of gemm_bf6_choose_nsplit where the
+// register-fed kernel runs unsplit in its place.
+struct LinPlan { size_t part, a6, xs, t, lpart, total, documented; int nsplit; };
 size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 LinPlan lin_plan(int M, int N, int K, int R) {
     LinPlan p{};
     const size_t rows = (size_t)((M + 255) / 256) * 256;
-    p.nsplit = convrot::gemm_bf6_choose_nsplit(M, N, K);
+    const int chosen = convrot::gemm_bf6_choose_nsplit(M, N, K);
     int bm = 0, bn = 0;
     convrot::gemm_bf6_direct_tile(M, N, K, &bm, &bn);
-    if (bm != 0) p.nsplit = 1;      // the direct kernel splits k inside its workgroups
+    p.nsplit = bm != 0 ? 1 : chosen;      // the direct kernel splits k inside its workgroups
+    auto region = [&](int nsplit) {
+        const size_t b = convrot::gemm_bf6_splitk_workspace(M, N, nsplit);
+        return al256(b > kSplitCounterBytes ? b : kSplitCounterBytes);
+    };
     p.part = 0;
-    const size_t split_bytes = convrot::gemm_bf6_splitk_workspace(M, N, convrot::gemm_bf6_choose_nsplit(M, N, K));
-    p.a6 = al256(split_bytes > kSplitCounterBytes ? split_bytes : kSplitCounterBytes);
+    p.a6 = region(p.nsplit);
     p.xs = p.a6 + al256(rows * (size_t)K / 4 * 3);
     p.t = p.xs + al256((size_t)M * 4);
     p.lpart = p.t + al256((size_t)M * R * 2);
     p.total = p.lpart + (R > 0 ? al256(convrot::lora_part_bytes(M, K, R)) : 0);
+    p.documented = p.total + region(chosen) - p.a6;
     return p;
 }
 }  // namespace
 
 API size_t cr_convrot_w4a4_linear_bf6_workspace(int M, int N, int K, int R) {
+    if (M <= 0 || N <= 0 || !bf6_k_ok(K) || R < 0) return 0;
+    return lin_plan(M, N, K, R).documented;
+}
+
+API size_t cr_convrot_w4a4_linear_bf6_min_workspace(int M, int N, int K, int R) {
     if (M <= 0 || N <= 0 || !bf6_k_ok(K) || R < 0) return 0;
     return lin_plan(M, N, K, R).total;
 }
@@ -493,7 +505,7 @@ API int cr_convrot_w4a4_linear_bf6_noalloc(const void* x, int in_dtype, const vo
     if (!linear_bf6_args_ok(in_dtype, bias_dtype, D, U, R, epilogue, M, N, K, G)) return -1;
     if (M == 0 || N == 0) return 0;
     const LinPlan p = lin_plan(M, N, K, R);
-    if (p.total > kScratchBytes) return -1;       // this shape needs more than the library's scratch
+    if (p.documented > kScratchBytes) return -1;  // the documented limit of this entry point
     void* ws = nullptr;
     hipError_t e = scratch_address(&ws);
     if (e != hipSuccess) return (int)e;

@@ -141,7 +141,7 @@ PyObject* w4a4(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const int M = (int)l.M, N = (int)l.N, K = (int)l.K;
     if (bf6 && cr_convrot_w4a4_linear_bf6_split(M, N, K)) Py_RETURN_NONE;
-    const size_t ws_bytes = bf6 ? cr_convrot_w4a4_linear_bf6_workspace(M, N, K, R)
+    const size_t ws_bytes = bf6 ? cr_convrot_w4a4_linear_bf6_min_workspace(M, N, K, R)
                                 : cr_convrot_w4a4_linear_packed_workspace(M, N, K, R);
     const int epi = l.xdt == 1 ? (a[5] == Py_True ? 2 : 1) : 0;
     int rc;

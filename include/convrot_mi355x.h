@@ -229,7 +229,9 @@ int cr_int4_convrot_gemm_bf6_splitk(const void* A6, const void* W6, const void* 
                                     void* out, int M, int N, int K, int epilogue, int nsplit,
                                     void* workspace, size_t workspace_bytes, void* stream);
 
-/* The library's k-split count for an M x N x K bf6 GEMM (1 = no split). */
+/* The library's k-split count for an M x N x K bf6 GEMM on staged tiles (1 = no split).
+ * The one-call linear runs the register-fed tiles of at most 256 rows unsplit instead:
+ * cr_convrot_w4a4_linear_bf6_split tells. */
 int cr_gemm_bf6_choose_nsplit(int M, int N, int K);
 
 /* The workgroup tile (*bm rows of A x *bn rows of B) of a bf6 GEMM launch of
@@ -250,13 +252,13 @@ size_t cr_gemm_bf6_splitk_workspace(int M, int N, int nsplit);
  * The whole W4A4 linear of the Linear replacement's forward in one call:
  *   out = epilogue(x_rot_quant @ W^T) [+ scale * (x @ D^T) @ U^T]
  * = cr_convrot_quant_bf6 on x, cr_lora_down when R > 0 (x bf16/f16), then the
- * bf6 GEMM (k-split when cr_gemm_bf6_choose_nsplit says so) with epilogue 0..2;
+ * bf6 GEMM (k-split when cr_convrot_w4a4_linear_bf6_split says so) with epilogue 0..2;
  * the same bits as those calls made one by one (here the LoRA partial sums are
  * added up by the rotate+quant kernel, in cr_lora_down's order).  W6 is the
  * weight in B6T (cr_int4_to_bf6), wscale f32 [N], bias [N] of bias_dtype (0 f32,
  * 1 bf16, 2 f16: the Linear keeps biases in fp16) or NULL, D
  * [R, K] / U [N, R] bf16 (R = 0: no LoRA).  The activation codes, scales, t and
- * split partials live in `workspace` (>= cr_convrot_w4a4_linear_bf6_workspace
+ * split partials live in `workspace` (>= cr_convrot_w4a4_linear_bf6_min_workspace
  * bytes, reused by the next call on the same stream).  K % 128 == 0,
  * K <= cr_max_quant_bf6_k().  No counterpart in the reference's ABI: it serves
  * the per-call sequence of _int4/__init__.py:94-138 with one FFI crossing.
@@ -271,8 +273,12 @@ int cr_convrot_w4a4_linear_bf6_f16(const void* x, int in_dtype, const void* W6, 
                                    int bias_dtype, const void* D, const void* U, int R, float scale, void* out, int M,
                                    int N, int K, int G, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Workspace bytes of cr_convrot_w4a4_linear_bf6 (and _f16) for this shape and LoRA rank. */
+/* Workspace bytes of cr_convrot_w4a4_linear_bf6 (and _f16) for this shape and LoRA rank.
+ * The calls use (and require) the first _min_workspace bytes: less where at most 256 rows
+ * run on register-fed tiles, which need none of the partials of
+ * cr_gemm_bf6_choose_nsplit's split (256 x 12288 -> 3072: 2.4 MB against 14.9). */
 size_t cr_convrot_w4a4_linear_bf6_workspace(int M, int N, int K, int R);
+size_t cr_convrot_w4a4_linear_bf6_min_workspace(int M, int N, int K, int R);
 
 /* 1 when the linear's GEMM splits k over workgroups, so that its workspace's
  * counters (the first 2048 bytes) have to be zero; 0: any workspace will do. */

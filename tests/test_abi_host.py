@@ -347,6 +347,25 @@ def test_split_choice_and_workspace(native):
     assert lib.cr_gemm_bf6_splitk_workspace(300, 300, 1) == 0
 
 
+def test_linear_reserves_only_what_it_uses(native):
+    """Unsplit linears of at most 256 rows hold counters, codes, scales and t, no
+    partials of a split that another kernel would run; split ones their partials."""
+    lib = native.load_library()
+    al = lambda v: (v + 255) // 256 * 256
+    for M, N, K in [(1, 3072, 12288), (64, 12288, 6144), (256, 3072, 12288), (256, 9216, 12288), (300, 3072, 12288),
+                    (512, 3072, 12288), (512, 3072, 3072), (4608, 3072, 12288)]:
+        for R in (0, 32):
+            rows, ns = (M + 255) // 256 * 256, lib.cr_gemm_bf6_choose_nsplit(M, N, K)
+            split = lib.cr_convrot_w4a4_linear_bf6_split(M, N, K)
+            region = max(2048, lib.cr_gemm_bf6_splitk_workspace(M, N, ns) if split else 0)
+            parts = max(0, lib.cr_lora_down_workspace(M, K, R) - 2048) if R else 0
+            want = al(region) + al(rows * K * 3 // 4) + al(4 * M) + al(2 * M * R) + al(parts)
+            got = lib.cr_convrot_w4a4_linear_bf6_min_workspace(M, N, K, R)
+            assert got == want <= lib.cr_convrot_w4a4_linear_bf6_workspace(M, N, K, R), (M, N, K, R)
+    assert lib.cr_convrot_w4a4_linear_bf6_min_workspace(256, 3072, 12288, 0) < 3 << 20
+    assert lib.cr_convrot_w4a4_linear_bf6_min_workspace(1, 1, 100, 0) == 0
+
+
 def test_tile_choice(native):
     """The workgroup tile and the split count are host arithmetic: 256 x 256
     on large grids; on small grids 128 x 192 exactly when 128 x 128 tiles

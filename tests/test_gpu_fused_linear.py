@@ -200,3 +200,32 @@ def test_strided_and_batched_inputs_equal_contiguous(backend, native, gpu, lora)
     xt = x3.reshape(B * T, K).t().contiguous().t()                # column-major storage of the same values
     yt = backend.convrot_w4a4_linear(xt, qw, ws, bias=b, convrot_groupsize=G, lora=pair)
     assert torch.equal(yt, y2)
+
+
+@pytest.mark.parametrize("M,N,K,R", [(1, 300, 6144, 0), (64, 3072, 6272, 32), (256, 3072, 12288, 64), (300, 3072, 6144, 32)])
+def test_linear_keeps_inside_its_workspace(backend, native, gpu, M, N, K, R):
+    """A workspace of exactly the bytes the call requires: the bytes behind it stay,
+    one byte less is refused."""
+    import ctypes
+    lib = native.load_library()
+    x = outlier_activations(M, K, seed=M).cuda()
+    qw, ws = backend.quantize_convrot_w4a4_weight(normal_weight(N, K, seed=N).cuda(), convrot_groupsize=64)
+    w6, b = backend.prepare_convrot_w4a4_weight_bf6(qw), normal_bias(N, seed=3).cuda()
+    D, U = _lora_pair(N, K, R, 5) if R else (None, None)
+    need = lib.cr_convrot_w4a4_linear_bf6_min_workspace(M, N, K, R)
+    buf = torch.zeros(need + 4096, dtype=torch.uint8, device="cuda")
+    buf[need:] = 0xA5
+    out = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    p = lambda t: None if t is None else t.data_ptr()
+
+    def call(nbytes):
+        return lib.cr_convrot_w4a4_linear_bf6(p(x), 1, p(w6), p(ws), p(b), 2, p(D), p(U), R, ctypes.c_float(1.0), p(out),
+                                              native.EPI_BF16, M, N, K, 64, p(buf), nbytes, native._stream(x.device))
+    assert call(need - 1) == -1 and call(need) == 0
+    assert bool((buf[need:] == 0xA5).all())
+    a6, xs = native.convrot_quant_bf6(x, 64)
+    if R:
+        want = native.int4_convrot_gemm_bf6_lora(a6, w6, xs, ws, b, native.lora_down(x, D), U, 1.0, native.EPI_BF16, nsplit=1)
+    else:
+        want = native.int4_convrot_gemm_bf6(a6, w6, xs, ws, b, native.EPI_BF16, nsplit=1)
+    assert torch.equal(out, want)
