@@ -7,15 +7,21 @@ from inputs import normal_bias, normal_weight, outlier_activations
 
 pytestmark = pytest.mark.gpu
 
-# register-fed, 128 x 128, 128 x 192, split 128 x 128, split 256 x 256 and 256 x 256 tiles; packed widths
-SHAPES = [(1, 300, 256), (100, 3001, 1152), (300, 2000, 384), (500, 9000, 256), (300, 3000, 6144), (2200, 3072, 6144),
-          (2300, 7000, 256), (65, 2999, 192), (1100, 4800, 320)]
+# every tile of the bf6 GEMM and the k split it runs with (None: packed widths)
+SHAPES = {(1, 300, 256): (32, 32, 1), (100, 3001, 1152): (64, 32, 1), (300, 2000, 384): (128, 128, 1),
+          (500, 9000, 256): (128, 192, 1), (300, 3000, 6144): (128, 128, 2), (1000, 3000, 12288): (128, 192, 2),
+          (2200, 3072, 6144): (256, 192, 1), (2300, 7000, 256): (256, 256, 1), (1000, 3200, 12288): (256, 256, 4),
+          (65, 2999, 192): None, (1100, 4800, 320): None}
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("R", [0, 32, 64])
 def test_w4a4_f16(backend, native, gpu, M, N, K, R):
     print(f"f16 out M={M} N={N} K={K} R={R}", flush=True)
+    if SHAPES[M, N, K] is not None:
+        split = native.load_library().cr_convrot_w4a4_linear_bf6_split(M, N, K)
+        ns = native.choose_nsplit_bf6(M, N, K) if split else 1
+        assert (*native.gemm_tile_bf6(M, N, K, ns), ns) == SHAPES[M, N, K]
     G = backend.pick_groupsize(K)
     x = outlier_activations(M, K, seed=M + 2).to(torch.float16).cuda()
     qw, s = backend.quantize_convrot_w4a4_weight(normal_weight(N, K, seed=N).cuda(), convrot_groupsize=G)
