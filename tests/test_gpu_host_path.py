@@ -158,3 +158,40 @@ def test_streams_and_threads(backend, native, gpu):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+@pytest.mark.parametrize("K,mode,R", [(512, "int4", 0), (512, "int4", 32), (1600, "int4", 0), (1600, "int4", 32), (512, "int8", 0)])
+def test_layers_take_the_host_path(backend, native, gpu, monkeypatch, K, mode, R):
+    """A loaded layer's forward (its codes a meta-device shape where a tile layout
+    is the operand) is answered by the host module in every activation type."""
+    import types
+    from test_gpu_footprint import _ops
+    host, taken = native.host_module(), []
+
+    def seen(name):
+        def call(*a):
+            y = getattr(host, name)(*a)
+            taken.append((name, y is not None))
+            return y
+        return call
+    monkeypatch.setattr(native, "_host", types.SimpleNamespace(w4a4=seen("w4a4"), w8a8=seen("w8a8")))
+    Ops, parent, N = _ops(), torch.nn.Module(), 384
+    parent.lin = Ops.Linear(K, N, bias=True)
+    Ops.int8_exact = {"lin"} if mode == "int8" else set()
+    try:
+        parent.load_state_dict({"lin.weight": normal_weight(N, K, seed=1).float(), "lin.bias": normal_bias(N, seed=2).float()},
+                               strict=False)
+    finally:
+        Ops.int8_exact = set()
+    lin = parent.lin
+    assert lin._qmode == mode
+    if R:
+        g = torch.Generator(device="cuda").manual_seed(1)
+        lin._dyn_fused = tuple((torch.randn(sh, generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+                               for sh in ((R, K), (N, R)))
+        lin._dyn_lora, lin._dyn_rest = [], []
+    types_ = (torch.bfloat16, torch.float16) if R else (torch.bfloat16, torch.float16, torch.float32)
+    for dt in types_:
+        y = lin(outlier_activations(48, K, seed=3).to(dt).cuda()[None])
+        assert y.shape == (1, 48, N) and y.dtype == dt
+    assert taken == [("w8a8" if mode == "int8" else "w4a4", True)] * len(types_)
