@@ -23,7 +23,9 @@ static long long up(int v, int t) { return (long long)((v + t - 1) / t); }
 // 3072 - / 13.8 / 13.2 / 15.5; 512 x 3072 -> 12288 and 2048 x 3072 -> 3072 20.5 on
 // 128 x 128 (384 workgroups); 512 x 12288 -> 3072 100.6 / 43.6, split in two
 // 29.3, in four 27.6 (64 x 64 44.6); 300 x 12288 -> 3072 (72 tiles)
-// 42.8, in two 28.3, in three 23.4, in four (288 workgroups) 28.7; 256 x 12288 ->
+// 42.8, in two 28.3, in three 23.4, in four (288 workgroups) 28.7 - what the rule
+// of one workgroup per CU follows, though it gives the 96 tiles of 512 rows two
+// ways where four are 1.7 us faster; 256 x 12288 ->
 // 3072 28.2 split in two, 20.7 in four, 23.4 on 64 x 64; 1024 x 12288 -> 3072 44.1, split in two 42.5; 1333 x
 // 2304 -> 6912 (594 workgroups) 25.6 against about 24 on 256 x 256.  Between
 // one and two 128 x 128 workgroups per CU, 256 x 128 tiles of four 128 x 64 waves
@@ -98,6 +100,7 @@ hipError_t gemm_i8t_launch(const int8_t* X, const int8_t* W, const float* xs, co
 // (1200 direct workgroups); 512 14.2 / 12.5 / 15.7; 1024 24.3 / 23.3 / 16.1 (304
 // of 128 x 128); 2048 48.9 / 34.3 / 30.9; 4096 92.0 / 56.2 / 46.4.  The 256 x 256
 // tiles staged through registers that these widths ran on took 42.2 at M = 1024.
+// The bound of 1536 direct workgroups was measured at this K alone.
 template <int EPI, bool LORA>
 static hipError_t p4_run(const uint8_t* A, const uint8_t* B, const float* xs, const float* ws, const void* bias,
                          int bias_dt, void* out, int M, int N, int K, const LoraArgs& la, hipStream_t st) {

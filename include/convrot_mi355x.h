@@ -21,9 +21,10 @@
  *     hipError_t of the launch (no device synchronisation).
  *   - packed int4 layout: int8 [rows, K/2], element 2j in the low nibble of
  *     byte j, 2j+1 in the high nibble (reference _int4/_codec.py:19-25).
- *   - workspaces (cr_lora_down, cr_int4_convrot_gemm_bf6_splitk,
- *     cr_convrot_w4a4_linear_bf6): bytes 0..2047 of every workspace hold the
- *     split counters of the bf6 GEMM.  They must be zero when a workspace is
+ *   - workspaces (cr_lora_down, cr_int4_convrot_gemm_bf6_splitk and the one-call
+ *     linears cr_convrot_w4a4_linear_bf6, _bf6_f16, _packed and
+ *     cr_convrot_w8a8_linear_i8t): bytes 0..2047 of every workspace hold the
+ *     split counters of the bf6 and W8A8 GEMMs.  They must be zero when a workspace is
  *     first used (clear them once after allocating it); every call leaves them
  *     zero, and no call writes anything else there, so one workspace can serve
  *     every entry point and shape in stream order.  The sizes returned by the

@@ -16,7 +16,7 @@ def sample(M, seed):
 
 
 # 32 x 32 tiles, 64 x 64, 128 x 128, split in four, three and two, 256 x 128, 256 x 256
-I8 = [(1, 449, 64), (33, 700, 1088), (200, 3000, 1152), (257, 3000, 320), (300, 3071, 64), (200, 3000, 6144),
+I8 = [(1, 449, 64), (33, 700, 1088), (200, 3000, 1152), (257, 3000, 320), (300, 3071, 64), (500, 3000, 320), (200, 3000, 6144),
       (300, 3000, 6144), (500, 3000, 6208), (2000, 3100, 1152), (1793, 4095, 64), (2100, 8000, 256)]
 
 
